@@ -39,25 +39,26 @@ __device__ __forceinline__ double2 cdiv(double2 a, double2 d)  // a / d
     return make_double2((a.x * d.x + a.y * d.y) / den, (a.y * d.x - a.x * d.y) / den);
 }
 
-// The search's constants on the device (FP64): c = C, ct = C^T [nel]; w[i*N+j] =
-// (i/hbar)(E_i - E_j); epsm[q] = eps - S_u of the ADO in slot q (eps in unused slots,
-// which the transform writes as zero).
+// One iteration's arguments: the state and the result (planes), the ordinary tables of a
+// handle (neighbour table, pf_same_sum = eps, tile flags, instance and bath class), and
+// epsm[q] = eps - S_u of the ADO in slot q (eps in unused slots, which are written as zero).
+// The constants with wave-uniform indices (C, C^T, w[i*N+j] = (i/hbar)(E_i - E_j) per
+// instance; gam and terms per class) are kernel arguments of their own, read with scalar
+// loads.
 struct TssArgs {
-    const double2* __restrict__ k;  // f_TSS(y), planes
-    double2* __restrict__ y;        // result, planes
-    const double2* __restrict__ c;  // [count][nel] (c, ct, w): the instance of each tile
-    const double2* __restrict__ ct;
-    const double2* __restrict__ w;
+    const double2* __restrict__ y;
+    double2* __restrict__ out;
+    const int2* __restrict__ nb;
+    const double2* __restrict__ pfss;
     const double2* __restrict__ epsm;
     const int32_t* __restrict__ q2u;        // < 0: padding or the zero slot, kept at zero
     const int32_t* __restrict__ tile_inst;  // instance of each tile (null: one instance)
+    const int32_t* __restrict__ tile_plus;
+    const int32_t* __restrict__ tile_class;  // bath class of each tile (null: one class)
     int64_t mp;
+    int32_t ntiles, zero_slot, xcd_chunk;
 };
 
-// y <- C^T [ (C k C^T) / D ] C for the 64 ADOs of a tile: wavefront i owns row i.
-// C k needs all rows of k (LDS); (C k) C^T and the division act on row i alone; C^T B
-// needs all rows of B (LDS again, after every wavefront has finished reading k); the
-// final right product acts on row i.
 // c * x (+ acc) with C's entries real when REALC (the eigenvectors of a real symmetric
 // H): two multiplies per product instead of four
 template <bool REALC>
@@ -68,66 +69,142 @@ __device__ __forceinline__ double2 cmac(double2 c, double2 x, double2 acc)
     return cfma(c, x, acc);
 }
 
-template <int N, bool REALC>
-__global__ __launch_bounds__(64 * N) void tss_transform(TssArgs a)
+// One iteration for the 64 ADOs of a tile (lane = ADO), one wavefront per column, then per
+// row, of the matrices.  Wavefront j evaluates column j of k = f_TSS(y) -- the "same" term
+// and the neighbour terms, no commutator -- and, holding the column in registers, column j
+// of C k.  The tile goes through LDS; wavefront i takes row i of C k, multiplies by C^T,
+// divides by D and multiplies by C, all within the row; the tile goes through LDS once
+// more (each wavefront overwrites the row that only it has read), and wavefront j stores
+// column j of C^T (B C).  So k and the products between never leave the CU, and the four
+// products cost two tile writes and two tile reads of LDS instead of a read of the whole
+// tile per matrix row for each left product.
+template <int N, int NT, bool REALC, bool PLUS>
+__device__ __forceinline__ void tss_tile(const TssArgs& a, const double2* __restrict__ gam,
+                                         const Term* __restrict__ terms, const double2* __restrict__ C,
+                                         const double2* __restrict__ CT, const double2* __restrict__ Wd, int tile,
+                                         double2* t)
 {
-    __shared__ double2 t[N * N * kTile];
     const int lane = threadIdx.x & 63;
-    const int i = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t q = (int64_t)blockIdx.x * kTile + lane;
-    const int64_t off = a.tile_inst ? (int64_t)a.tile_inst[blockIdx.x] * N * N : 0;
-    const double2* __restrict__ C = a.c + off;
-    const double2* __restrict__ CT = a.ct + off;
-    const double2* __restrict__ Wd = a.w + off;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t mp = a.mp;
+    const int64_t q = (int64_t)tile * kTile + lane;
+    const double2 S = a.pfss[q];
+    const double sq_lane = sqrt((double)lane);  // sqrt(n), n = 0..63, one value per lane
+    // gathers as raw buffer loads, one resource per element plane whose range ends at the
+    // zero slot: an edge to it returns zero without a memory request
+    const int nrec = a.zero_slot * (int)sizeof(double2);
+    auto gather = [&](__amdgpu_buffer_rsrc_t rsrc, uint32_t idx) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, idx * (uint32_t)sizeof(double2), 0, 0);
+        return make_double2(__hiloint2double((int)v[1], (int)v[0]), __hiloint2double((int)v[3], (int)v[2]));
+    };
+    // offsets the compiler cannot see through keep the (scalar, cached) loads of the
+    // uniform constants next to the row or column that uses them: hoisted together they
+    // would need several times the scalar registers
+    auto opaque = [](const double2* p) {
+        int z;
+        asm volatile("s_mov_b32 %0, 0" : "=s"(z));
+        return p + z;
+    };
+    double2 r[N];
 #pragma unroll
-    for (int j = 0; j < N; ++j)
-        t[(i * N + j) * kTile + lane] = a.k[(int64_t)(i * N + j) * a.mp + q];
-    __syncthreads();
-    double2 r[N], s[N];
+    for (int i = 0; i < N; ++i) {  // r = column w of k
+        const int e = i * N + w;
+        const double2* plane = a.y + (int64_t)e * mp;
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)plane, (short)0, nrec, 0x00020000);
+        int2 nbv[NT];
+        double2 xp[NT], xm[NT];
 #pragma unroll
-    for (int j = 0; j < N; ++j)
-        r[j] = make_double2(0.0, 0.0);
+        for (int k = 0; k < NT; ++k)
+            nbv[k] = a.nb[(int64_t)terms[e * NT + k].mode * mp + q];
 #pragma unroll
-    for (int m = 0; m < N; ++m) {  // r = row i of C k
-        const double2 cim = C[i * N + m];
+        for (int k = 0; k < NT; ++k) {
+            if constexpr (PLUS)
+                xp[k] = gather(rsrc, (uint32_t)nbv[k].x >> 6);
+            xm[k] = gather(rsrc, (uint32_t)nbv[k].y);
+        }
+        const double2 g = gam[e];
+        double2 f = cfma(make_double2(S.x + g.x, S.y + g.y), plane[q], make_double2(0.0, 0.0));
 #pragma unroll
-        for (int j = 0; j < N; ++j)
-            r[j] = cmac<REALC>(cim, t[(m * N + j) * kTile + lane], r[j]);
+        for (int k = 0; k < NT; ++k) {
+            const Term tm = terms[e * NT + k];
+            const int v = nbv[k].x & 63;
+            if constexpr (PLUS) {
+                const double cp = tm.plus_c * lane_value(sq_lane, v + 1);
+                f.x = fma(-cp, xp[k].y, f.x);
+                f.y = fma(cp, xp[k].x, f.y);
+            }
+            const double sm = lane_value(sq_lane, v);
+            f = cfma(tm.minus_c, make_double2(sm * xm[k].x, sm * xm[k].y), f);
+        }
+        r[i] = f;
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {  // column w of C k
+        const double2* Ci = opaque(C) + i * N;
+        double2 v = make_double2(0.0, 0.0);
+#pragma unroll
+        for (int m = 0; m < N; ++m)
+            v = cmac<REALC>(Ci[m], r[m], v);
+        t[(i * N + w) * kTile + lane] = v;
     }
     const double2 em = a.epsm[q];
     const bool pad = a.q2u[q] < 0;
+    __syncthreads();
+    double2 s[N];
 #pragma unroll
-    for (int j = 0; j < N; ++j) {  // s = row i of (C k C^T) / D
+    for (int m = 0; m < N; ++m)
+        r[m] = t[(w * N + m) * kTile + lane];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {  // s = row w of (C k C^T) / D
+        const double2* Cj = opaque(C) + j * N;
         double2 v = make_double2(0.0, 0.0);
 #pragma unroll
         for (int m = 0; m < N; ++m)
-            v = cmac<REALC>(CT[m * N + j], r[m], v);
-        const double2 wij = Wd[i * N + j];
+            v = cmac<REALC>(Cj[m], r[m], v);  // CT[m][j]
+        const double2 wij = Wd[w * N + j];
         s[j] = cdiv(v, make_double2(wij.x + em.x, wij.y + em.y));
     }
-    __syncthreads();  // every wavefront is done with k
 #pragma unroll
-    for (int j = 0; j < N; ++j)
-        t[(i * N + j) * kTile + lane] = s[j];
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < N; ++j)
-        r[j] = make_double2(0.0, 0.0);
-#pragma unroll
-    for (int m = 0; m < N; ++m) {  // r = row i of C^T B
-        const double2 ctim = CT[i * N + m];
-#pragma unroll
-        for (int j = 0; j < N; ++j)
-            r[j] = cmac<REALC>(ctim, t[(m * N + j) * kTile + lane], r[j]);
-    }
-#pragma unroll
-    for (int j = 0; j < N; ++j) {  // row i of C^T B C
+    for (int j = 0; j < N; ++j) {  // row w of B C
+        const double2* CTj = opaque(CT) + j * N;
         double2 v = make_double2(0.0, 0.0);
 #pragma unroll
         for (int m = 0; m < N; ++m)
-            v = cmac<REALC>(C[m * N + j], r[m], v);
-        a.y[(int64_t)(i * N + j) * a.mp + q] = pad ? make_double2(0.0, 0.0) : v;
+            v = cmac<REALC>(CTj[m], s[m], v);  // C[m][j]
+        t[(w * N + j) * kTile + lane] = v;
     }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < N; ++m)
+        r[m] = t[(m * N + w) * kTile + lane];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {  // column w of C^T (B C)
+        const double2* CTi = opaque(CT) + i * N;
+        double2 v = make_double2(0.0, 0.0);
+#pragma unroll
+        for (int m = 0; m < N; ++m)
+            v = cmac<REALC>(CTi[m], r[m], v);
+        nt_store<double>(pad ? make_double2(0.0, 0.0) : v, a.out + (int64_t)(i * N + w) * mp + q);
+    }
+}
+
+template <int N, int NT, bool REALC>
+__global__ __launch_bounds__(64 * N) void tss_iteration(TssArgs a, const double2* __restrict__ gam,
+                                                        const Term* __restrict__ terms,
+                                                        const double2* __restrict__ c,
+                                                        const double2* __restrict__ ct,
+                                                        const double2* __restrict__ wd)
+{
+    __shared__ double2 t[N * N * kTile];
+    const int tile = xcd_tile(blockIdx.x, a.ntiles, a.xcd_chunk);
+    const int64_t off = a.tile_inst ? (int64_t)a.tile_inst[tile] * N * N : 0;
+    const int cls = a.tile_class ? a.tile_class[tile] : 0;
+    gam += cls * (N * N);
+    terms += cls * (N * N * NT);
+    if (a.tile_plus[tile] != 0)
+        tss_tile<N, NT, REALC, true>(a, gam, terms, c + off, ct + off, wd + off, tile, t);
+    else
+        tss_tile<N, NT, REALC, false>(a, gam, terms, c + off, ct + off, wd + off, tile, t);
 }
 
 // 8 < N <= 32, one pass, thread = (element e, slot q):
@@ -166,13 +243,27 @@ __global__ void tss_pass(const double2* __restrict__ in, double2* __restrict__ o
     out[t] = q2u[q] < 0 ? make_double2(0.0, 0.0) : v;
 }
 
-template <int N>
-void launch_transform(heom_handle* h, const TssArgs& a, bool real_c)
+template <int N, int NT>
+void launch_iteration_t(heom_handle* h, const TssArgs& a)
 {
-    if (real_c)
-        hipLaunchKernelGGL((tss_transform<N, true>), dim3(h->ntiles), dim3(64 * N), 0, h->stream, a);
+    const TssState& T = *h->tss;
+    const dim3 grid(h->ntiles), block(64 * N);
+    if (T.real_c)
+        hipLaunchKernelGGL((tss_iteration<N, NT, true>), grid, block, 0, h->stream, a, h->gam.p, h->terms.p, T.c.p,
+                           T.ct.p, T.w.p);
     else
-        hipLaunchKernelGGL((tss_transform<N, false>), dim3(h->ntiles), dim3(64 * N), 0, h->stream, a);
+        hipLaunchKernelGGL((tss_iteration<N, NT, false>), grid, block, 0, h->stream, a, h->gam.p, h->terms.p, T.c.p,
+                           T.ct.p, T.w.p);
+}
+
+template <int N>
+void launch_iteration(heom_handle* h, const TssArgs& a)
+{
+    switch (h->term_slots) {
+    case 2: launch_iteration_t<N, 2>(h, a); break;
+    case 4: launch_iteration_t<N, 4>(h, a); break;
+    default: launch_iteration_t<N, 8>(h, a); break;
+    }
 }
 
 void check_tss(heom_handle* h)
@@ -318,32 +409,39 @@ int heom_tss_step(heom_handle* h, int64_t n)
             raise(HEOM_E_INVALID, "n must be >= 0");
         const TssState& T = *h->tss;
         const int N = h->N;
-        double2* y = h->y.as<double2>();
-        double2* ya = h->ya.as<double2>();
-        double2* yb = h->yb.as<double2>();
         const int32_t* ti = h->count > 1 ? h->tile_inst.p : nullptr;
-        TssArgs a{ya, y, T.c.p, T.ct.p, T.w.p, T.epsm.p, h->q2u.p, ti, h->Mp};
         const int64_t total = (int64_t)h->nel * h->Mp;
         const dim3 pgrid(blocks_for(total, 256)), pblock(256);
         for (int64_t s = 0; s < n; ++s) {
-            launch_stage_buffers(h, 0, h->y.p, h->y.p, h->pbuf.p, h->ya.p, 0.0, false, false);
-            switch (N) {
-            case 1: launch_transform<1>(h, a, T.real_c); break;
-            case 2: launch_transform<2>(h, a, T.real_c); break;
-            case 3: launch_transform<3>(h, a, T.real_c); break;
-            case 4: launch_transform<4>(h, a, T.real_c); break;
-            case 5: launch_transform<5>(h, a, T.real_c); break;
-            case 6: launch_transform<6>(h, a, T.real_c); break;
-            case 7: launch_transform<7>(h, a, T.real_c); break;
-            case 8: launch_transform<8>(h, a, T.real_c); break;
-            default:
-                // C k -> yb, (. C^T) / D -> ya, C^T . -> yb, . C -> y, in the reference's order
-                hipLaunchKernelGGL(tss_pass, pgrid, pblock, 0, h->stream, ya, yb, T.c.p, nullptr, nullptr, h->q2u.p, ti, h->Mp, N, 1);
-                hipLaunchKernelGGL(tss_pass, pgrid, pblock, 0, h->stream, yb, ya, T.ct.p, T.w.p, T.epsm.p, h->q2u.p, ti, h->Mp, N, 0);
-                hipLaunchKernelGGL(tss_pass, pgrid, pblock, 0, h->stream, ya, yb, T.ct.p, nullptr, nullptr, h->q2u.p, ti, h->Mp, N, 1);
-                hipLaunchKernelGGL(tss_pass, pgrid, pblock, 0, h->stream, yb, y, T.c.p, nullptr, nullptr, h->q2u.p, ti, h->Mp, N, 0);
-                break;
+            if (N <= kMaxStates) {
+                // y -> ya, then the two exchange their places
+                const TssArgs a{h->y.as<double2>(), h->ya.as<double2>(), h->nb.p, h->pfss.p, T.epsm.p, h->q2u.p, ti,
+                                h->tile_plus.p, h->uniform ? nullptr : h->tile_class.p, h->Mp, h->ntiles,
+                                h->zero_slot, h->xcd_chunk};
+                switch (N) {
+                case 1: launch_iteration<1>(h, a); break;
+                case 2: launch_iteration<2>(h, a); break;
+                case 3: launch_iteration<3>(h, a); break;
+                case 4: launch_iteration<4>(h, a); break;
+                case 5: launch_iteration<5>(h, a); break;
+                case 6: launch_iteration<6>(h, a); break;
+                case 7: launch_iteration<7>(h, a); break;
+                default: launch_iteration<8>(h, a); break;
+                }
+                HIPC(hipGetLastError());
+                std::swap(h->y.p, h->ya.p);
+                h->timing.rhs_launches += 1;
+                continue;
             }
+            double2* y = h->y.as<double2>();
+            double2* ya = h->ya.as<double2>();
+            double2* yb = h->yb.as<double2>();
+            launch_stage_buffers(h, 0, h->y.p, h->y.p, h->pbuf.p, h->ya.p, 0.0, false, false);
+            // C k -> yb, (. C^T) / D -> ya, C^T . -> yb, . C -> y, in the reference's order
+            hipLaunchKernelGGL(tss_pass, pgrid, pblock, 0, h->stream, ya, yb, T.c.p, nullptr, nullptr, h->q2u.p, ti, h->Mp, N, 1);
+            hipLaunchKernelGGL(tss_pass, pgrid, pblock, 0, h->stream, yb, ya, T.ct.p, T.w.p, T.epsm.p, h->q2u.p, ti, h->Mp, N, 0);
+            hipLaunchKernelGGL(tss_pass, pgrid, pblock, 0, h->stream, ya, yb, T.ct.p, nullptr, nullptr, h->q2u.p, ti, h->Mp, N, 1);
+            hipLaunchKernelGGL(tss_pass, pgrid, pblock, 0, h->stream, yb, y, T.c.p, nullptr, nullptr, h->q2u.p, ti, h->Mp, N, 0);
             HIPC(hipGetLastError());
         }
     });
