@@ -117,6 +117,11 @@ struct TssState {
     DevBuf<double2> w;      // (i/hbar)(E_i - E_j) [count][nel]
     DevBuf<double2> epsm;   // eps - S_u per slot [Mp]
     bool real_c = false;    // C has no imaginary parts (real symmetric H)
+    // N <= 8: the real parts of C and C^T, and the element constants in column-major order
+    DevBuf<double> cr, ctr;           // [count][nel]
+    DevBuf<double2> gam;              // [classes][N columns][N]
+    DevBuf<heom_hip::Term> terms;     // [classes][N columns][N][term slots]
+    DevBuf<int32_t> modes;            // the terms' modes alone
 };
 
 }  // namespace heom_rt

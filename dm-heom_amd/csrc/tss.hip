@@ -59,15 +59,13 @@ struct TssArgs {
     int32_t ntiles, zero_slot, xcd_chunk;
 };
 
-// c * x (+ acc) with C's entries real when REALC (the eigenvectors of a real symmetric
-// H): two multiplies per product instead of four
-template <bool REALC>
-__device__ __forceinline__ double2 cmac(double2 c, double2 x, double2 acc)
+// c * x (+ acc): C's entries are real for a real symmetric H (two multiplies per product
+// instead of four, and half the scalar loads), complex otherwise
+__device__ __forceinline__ double2 cmac(double c, double2 x, double2 acc)
 {
-    if (REALC)
-        return make_double2(fma(c.x, x.x, acc.x), fma(c.x, x.y, acc.y));
-    return cfma(c, x, acc);
+    return make_double2(fma(c, x.x, acc.x), fma(c, x.y, acc.y));
 }
+__device__ __forceinline__ double2 cmac(double2 c, double2 x, double2 acc) { return cfma(c, x, acc); }
 
 // One iteration for the 64 ADOs of a tile (lane = ADO), one wavefront per column, then per
 // row, of the matrices.  Wavefront j evaluates column j of k = f_TSS(y) -- the "same" term
@@ -78,11 +76,11 @@ __device__ __forceinline__ double2 cmac(double2 c, double2 x, double2 acc)
 // column j of C^T (B C).  So k and the products between never leave the CU, and the four
 // products cost two tile writes and two tile reads of LDS instead of a read of the whole
 // tile per matrix row for each left product.
-template <int N, int NT, bool REALC, bool PLUS>
+template <int N, int NT, typename TC, bool PLUS>
 __device__ __forceinline__ void tss_tile(const TssArgs& a, const double2* __restrict__ gam,
-                                         const Term* __restrict__ terms, const double2* __restrict__ C,
-                                         const double2* __restrict__ CT, const double2* __restrict__ Wd, int tile,
-                                         double2* t)
+                                         const Term* __restrict__ terms, const int32_t* __restrict__ modes,
+                                         const TC* __restrict__ C, const TC* __restrict__ CT,
+                                         const double2* __restrict__ Wd, int tile, double2* t)
 {
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -100,51 +98,78 @@ __device__ __forceinline__ void tss_tile(const TssArgs& a, const double2* __rest
     // offsets the compiler cannot see through keep the (scalar, cached) loads of the
     // uniform constants next to the row or column that uses them: hoisted together they
     // would need several times the scalar registers
-    auto opaque = [](const double2* p) {
+    auto opaque = [](const auto* p) {
         int z;
         asm volatile("s_mov_b32 %0, 0" : "=s"(z));
         return p + z;
     };
+    // the wavefront's constants are contiguous (column-major elements)
+    gam += w * N;
+    terms += w * N * NT;
+    modes += w * N * NT;
+    // The table entries of a batch of elements are requested together, and where the
+    // registers allow (two workgroups of 8 wavefronts per CU: 128) an element's gathers and
+    // own value go out before the previous element's are summed.
+    constexpr bool AHEAD = NT * (PLUS ? 2 : 1) <= 4;
+    constexpr int HB = NT <= 2 ? N : NT <= 4 ? (N + 1) / 2 : 1;
     double2 r[N];
 #pragma unroll
-    for (int i = 0; i < N; ++i) {  // r = column w of k
-        const int e = i * N + w;
-        const double2* plane = a.y + (int64_t)e * mp;
-        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)plane, (short)0, nrec, 0x00020000);
-        int2 nbv[NT];
-        double2 xp[NT], xm[NT];
+    for (int i0 = 0; i0 < N; i0 += HB) {  // r = column w of k
+        int2 nbv[HB][NT];
 #pragma unroll
-        for (int k = 0; k < NT; ++k)
-            nbv[k] = a.nb[(int64_t)terms[e * NT + k].mode * mp + q];
+        for (int i = i0; i < i0 + HB && i < N; ++i)
 #pragma unroll
-        for (int k = 0; k < NT; ++k) {
-            if constexpr (PLUS)
-                xp[k] = gather(rsrc, (uint32_t)nbv[k].x >> 6);
-            xm[k] = gather(rsrc, (uint32_t)nbv[k].y);
-        }
-        const double2 g = gam[e];
-        double2 f = cfma(make_double2(S.x + g.x, S.y + g.y), plane[q], make_double2(0.0, 0.0));
+            for (int k = 0; k < NT; ++k)
+                nbv[i - i0][k] = a.nb[(int64_t)modes[i * NT + k] * mp + q];
+        double2 xp[AHEAD ? 2 : 1][NT], xm[AHEAD ? 2 : 1][NT], own[AHEAD ? 2 : 1];
+        auto load = [&](int i, int b) {
+            const double2* plane = a.y + (int64_t)(i * N + w) * mp;
+            const __amdgpu_buffer_rsrc_t rsrc =
+                __builtin_amdgcn_make_buffer_rsrc((void*)plane, (short)0, nrec, 0x00020000);
+            own[b] = plane[q];
 #pragma unroll
-        for (int k = 0; k < NT; ++k) {
-            const Term tm = terms[e * NT + k];
-            const int v = nbv[k].x & 63;
-            if constexpr (PLUS) {
-                const double cp = tm.plus_c * lane_value(sq_lane, v + 1);
-                f.x = fma(-cp, xp[k].y, f.x);
-                f.y = fma(cp, xp[k].x, f.y);
+            for (int k = 0; k < NT; ++k) {
+                if constexpr (PLUS)
+                    xp[b][k] = gather(rsrc, (uint32_t)nbv[i - i0][k].x >> 6);
+                xm[b][k] = gather(rsrc, (uint32_t)nbv[i - i0][k].y);
             }
-            const double sm = lane_value(sq_lane, v);
-            f = cfma(tm.minus_c, make_double2(sm * xm[k].x, sm * xm[k].y), f);
+        };
+        if (AHEAD)
+            load(i0, 0);
+#pragma unroll
+        for (int i = i0; i < i0 + HB && i < N; ++i) {
+            const int b = AHEAD ? (i - i0) & 1 : 0;
+            __builtin_amdgcn_sched_barrier(0);
+            if (!AHEAD)
+                load(i, 0);
+            else if (i + 1 < i0 + HB && i + 1 < N)
+                load(i + 1, 1 - b);
+            const Term* te = opaque(terms) + i * NT;
+            const double2 g = opaque(gam)[i];
+            double2 f = cfma(make_double2(S.x + g.x, S.y + g.y), own[b], make_double2(0.0, 0.0));
+#pragma unroll
+            for (int k = 0; k < NT; ++k) {
+                const int v = nbv[i - i0][k].x & 63;
+                if constexpr (PLUS) {
+                    const double cp = te[k].plus_c * lane_value(sq_lane, v + 1);
+                    f.x = fma(-cp, xp[b][k].y, f.x);
+                    f.y = fma(cp, xp[b][k].x, f.y);
+                }
+                const double sm = lane_value(sq_lane, v);
+                f = cfma(te[k].minus_c, make_double2(sm * xm[b][k].x, sm * xm[b][k].y), f);
+            }
+            // the sum is formed here, before the next element's gathers replace this one's
+            asm volatile("" : "+v"(f.x), "+v"(f.y));
+            r[i] = f;
         }
-        r[i] = f;
     }
 #pragma unroll
     for (int i = 0; i < N; ++i) {  // column w of C k
-        const double2* Ci = opaque(C) + i * N;
+        const TC* Ci = opaque(C) + i * N;
         double2 v = make_double2(0.0, 0.0);
 #pragma unroll
         for (int m = 0; m < N; ++m)
-            v = cmac<REALC>(Ci[m], r[m], v);
+            v = cmac(Ci[m], r[m], v);
         t[(i * N + w) * kTile + lane] = v;
     }
     const double2 em = a.epsm[q];
@@ -156,21 +181,21 @@ __device__ __forceinline__ void tss_tile(const TssArgs& a, const double2* __rest
         r[m] = t[(w * N + m) * kTile + lane];
 #pragma unroll
     for (int j = 0; j < N; ++j) {  // s = row w of (C k C^T) / D
-        const double2* Cj = opaque(C) + j * N;
+        const TC* Cj = opaque(C) + j * N;
         double2 v = make_double2(0.0, 0.0);
 #pragma unroll
         for (int m = 0; m < N; ++m)
-            v = cmac<REALC>(Cj[m], r[m], v);  // CT[m][j]
+            v = cmac(Cj[m], r[m], v);  // CT[m][j]
         const double2 wij = Wd[w * N + j];
         s[j] = cdiv(v, make_double2(wij.x + em.x, wij.y + em.y));
     }
 #pragma unroll
     for (int j = 0; j < N; ++j) {  // row w of B C
-        const double2* CTj = opaque(CT) + j * N;
+        const TC* CTj = opaque(CT) + j * N;
         double2 v = make_double2(0.0, 0.0);
 #pragma unroll
         for (int m = 0; m < N; ++m)
-            v = cmac<REALC>(CTj[m], s[m], v);  // C[m][j]
+            v = cmac(CTj[m], s[m], v);  // C[m][j]
         t[(w * N + j) * kTile + lane] = v;
     }
     __syncthreads();
@@ -179,21 +204,20 @@ __device__ __forceinline__ void tss_tile(const TssArgs& a, const double2* __rest
         r[m] = t[(m * N + w) * kTile + lane];
 #pragma unroll
     for (int i = 0; i < N; ++i) {  // column w of C^T (B C)
-        const double2* CTi = opaque(CT) + i * N;
+        const TC* CTi = opaque(CT) + i * N;
         double2 v = make_double2(0.0, 0.0);
 #pragma unroll
         for (int m = 0; m < N; ++m)
-            v = cmac<REALC>(CTi[m], r[m], v);
+            v = cmac(CTi[m], r[m], v);
         nt_store<double>(pad ? make_double2(0.0, 0.0) : v, a.out + (int64_t)(i * N + w) * mp + q);
     }
 }
 
-template <int N, int NT, bool REALC>
+template <int N, int NT, typename TC>
 __global__ __launch_bounds__(64 * N) void tss_iteration(TssArgs a, const double2* __restrict__ gam,
                                                         const Term* __restrict__ terms,
-                                                        const double2* __restrict__ c,
-                                                        const double2* __restrict__ ct,
-                                                        const double2* __restrict__ wd)
+                                                        const int32_t* __restrict__ modes, const TC* __restrict__ c,
+                                                        const TC* __restrict__ ct, const double2* __restrict__ wd)
 {
     __shared__ double2 t[N * N * kTile];
     const int tile = xcd_tile(blockIdx.x, a.ntiles, a.xcd_chunk);
@@ -201,10 +225,11 @@ __global__ __launch_bounds__(64 * N) void tss_iteration(TssArgs a, const double2
     const int cls = a.tile_class ? a.tile_class[tile] : 0;
     gam += cls * (N * N);
     terms += cls * (N * N * NT);
+    modes += cls * (N * N * NT);
     if (a.tile_plus[tile] != 0)
-        tss_tile<N, NT, REALC, true>(a, gam, terms, c + off, ct + off, wd + off, tile, t);
+        tss_tile<N, NT, TC, true>(a, gam, terms, modes, c + off, ct + off, wd + off, tile, t);
     else
-        tss_tile<N, NT, REALC, false>(a, gam, terms, c + off, ct + off, wd + off, tile, t);
+        tss_tile<N, NT, TC, false>(a, gam, terms, modes, c + off, ct + off, wd + off, tile, t);
 }
 
 // 8 < N <= 32, one pass, thread = (element e, slot q):
@@ -249,11 +274,11 @@ void launch_iteration_t(heom_handle* h, const TssArgs& a)
     const TssState& T = *h->tss;
     const dim3 grid(h->ntiles), block(64 * N);
     if (T.real_c)
-        hipLaunchKernelGGL((tss_iteration<N, NT, true>), grid, block, 0, h->stream, a, h->gam.p, h->terms.p, T.c.p,
-                           T.ct.p, T.w.p);
+        hipLaunchKernelGGL((tss_iteration<N, NT, double>), grid, block, 0, h->stream, a, T.gam.p, T.terms.p, T.modes.p,
+                           T.cr.p, T.ctr.p, T.w.p);
     else
-        hipLaunchKernelGGL((tss_iteration<N, NT, false>), grid, block, 0, h->stream, a, h->gam.p, h->terms.p, T.c.p,
-                           T.ct.p, T.w.p);
+        hipLaunchKernelGGL((tss_iteration<N, NT, double2>), grid, block, 0, h->stream, a, T.gam.p, T.terms.p,
+                           T.modes.p, T.c.p, T.ct.p, T.w.p);
 }
 
 template <int N>
@@ -372,15 +397,48 @@ int heom_create_tss_batch(const heom_desc* descs, int32_t count, const double* c
             em[(size_t)q] = make_double2(eps.real() - descs[k].pf_same_sum[2 * lu],
                                          eps.imag() - descs[k].pf_same_sum[2 * lu + 1]);
         }
-        auto up = [&](DevBuf<double2>& b, const std::vector<double2>& v) {
+        auto up = [&](auto& b, const auto& v) {  // complete on return: v may be a temporary
             b.alloc(v.size());
-            HIPC(hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(double2), hipMemcpyHostToDevice, h->stream));
+            HIPC(hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, h->stream));
+            HIPC(hipStreamSynchronize(h->stream));
         };
         T->real_c = true;
         for (const double2& x : cv)
             T->real_c = T->real_c && x.y == 0.0;
         up(T->c, cv);
         up(T->ct, ctv);
+        if (N <= kMaxStates) {
+            // real parts of C and C^T, and the element constants in column-major order
+            // (a wavefront of the iteration kernel evaluates one column)
+            std::vector<double> cr(cv.size()), ctr(cv.size());
+            for (size_t e = 0; e < cv.size(); ++e) {
+                cr[e] = cv[e].x;
+                ctr[e] = ctv[e].x;
+            }
+            const int NT = h->term_slots, classes = (int)h->classes.size();
+            std::vector<double2> gam((size_t)classes * nel), gam_c(gam.size());
+            std::vector<Term> terms((size_t)classes * nel * NT), terms_c(terms.size());
+            std::vector<int32_t> modes(terms.size());
+            HIPC(hipMemcpyAsync(gam.data(), h->gam.p, gam.size() * sizeof(double2), hipMemcpyDeviceToHost, h->stream));
+            HIPC(hipMemcpyAsync(terms.data(), h->terms.p, terms.size() * sizeof(Term), hipMemcpyDeviceToHost,
+                                h->stream));
+            HIPC(hipStreamSynchronize(h->stream));
+            for (int cl = 0; cl < classes; ++cl)
+                for (int i = 0; i < N; ++i)
+                    for (int j = 0; j < N; ++j) {
+                        const size_t from = (size_t)cl * nel + i * N + j, to = (size_t)cl * nel + j * N + i;
+                        gam_c[to] = gam[from];
+                        for (int k = 0; k < NT; ++k) {
+                            terms_c[to * NT + k] = terms[from * NT + k];
+                            modes[to * NT + k] = terms[from * NT + k].mode;
+                        }
+                    }
+            up(T->cr, cr);
+            up(T->ctr, ctr);
+            up(T->gam, gam_c);
+            up(T->terms, terms_c);
+            up(T->modes, modes);
+        }
         up(T->w, wv);
         up(T->epsm, em);
         HIPC(hipStreamSynchronize(h->stream));
