@@ -151,7 +151,7 @@ struct heom_handle {
     bool pipelined = false;  // stage_pipelined.hip (persistent) instead of stage_kernel.hip
     int pipe_wgs = 0;        // its workgroups: one per CU, a multiple of the XCD count
     int xcd_chunk = 1;       // tiles per XCD chunk of the stage kernels' tile order
-    int wide_ados = 0;       // N > 8: ADOs per workgroup of the wide kernel (0 = the most that fit)
+    int wide_ados = 0;       // N > 8: wavefronts (ADOs at a time) per workgroup (0 = the default)
     int tile_split = 1;      // tile kernel: workgroups per 64-ADO tile (1, 2 or 4)
     bool paired = false;     // complex64 planes in the paired layout (stage_pair.hip)
     int pair_slots = 0;      // neighbour terms per plane of the paired layout (0: not possible)
@@ -190,6 +190,13 @@ struct heom_handle {
     DevBuf<float2> pfss32, hs32, gam32;
     DevBuf<TermT<float>> terms32;
     DevBuf<heom_hip::PairTerm> pterms;  // [classes][pair_planes(N)][pair_slots]
+    // N > 8: the neighbour terms by mode (WideTables), [classes][W][wide_len]
+    DevBuf<Term> wterms;
+    DevBuf<TermT<float>> wterms32;
+    DevBuf<uint32_t> wwhere;
+    DevBuf<uint16_t> wplace;  // [N*N]
+    DevBuf<int32_t> tile_order;  // tiles with plus neighbours first
+    int wide_len = 0;
     int S = 0;                    // tier-0/1 ADOs
     std::vector<int32_t> sp_top;  // [count] tier-0/1 index of each top
     std::vector<int64_t> sp_uid;  // [S] global uid
@@ -220,6 +227,14 @@ struct heom_handle {
     std::unique_ptr<heom_rt::TssState> tss;
 
     bool fp32() const { return prec == HEOM_PRECISION_FP32; }
+    template <typename R>
+    heom_hip::WideTables<R> wide_tables() const
+    {
+        if constexpr (sizeof(R) == sizeof(double))
+            return {wterms.p, wwhere.p, tile_order.p, wplace.p, W, wide_len};
+        else
+            return {wterms32.p, wwhere.p, tile_order.p, wplace.p, W, wide_len};
+    }
     size_t cbytes() const { return fp32() ? sizeof(float2) : sizeof(double2); }
 
     heom_handle();
@@ -252,6 +267,9 @@ inline unsigned blocks_for(int64_t n, int threads) { return (unsigned)((n + thre
 // top_src ([count][N*N], stage 4 only) is added to the output at each instance's top ADO
 void launch_stage_buffers(heom_handle* h, int stage, const void* yin, const void* y0, void* pbuf, void* yout,
                           double c1, bool reverse, bool adjoint, const double2* top_src = nullptr);
+// the arguments of such a stage in FP64
+heom_hip::StageArgsT<double> stage_args64(heom_handle* h, const void* yin, const void* y0, void* pbuf, void* yout,
+                                          double c1, bool reverse);
 // builds the device layout of count instances into a fresh handle (heom_create_batch)
 void create_batch(heom_handle* h, const heom_desc* d, int count);
 // raises HEOM_E_UNSUPPORTED for `what` on a thermal-state-search handle

@@ -7,7 +7,8 @@
 //     fifths of all neighbour reads land within 30k ADOs, against one in twenty in the
 //     reference's layer order, so most of them are served from L2 / MALL.
 //   * State planes are structure-of-arrays by matrix element: Y[e * Mp + q] holds
-//     element e = i*N + j of ADO q as a double2 (re, im), or a float2.  Mp = M + 1 rounded up to a
+//     element e = i*N + j of ADO q as a double2 (re, im), or a float2; with more than eight
+//     states the state is matrix-major (wide_pos).  Mp = M + 1 rounded up to a
 //     multiple of 64.  Slot M (and every padding slot) is an ADO with no neighbours
 //     that stays exactly zero; edges that do not exist, or whose target is masked,
 //     point at slot M ("zero slot"), so gathers need no per-lane branches.
@@ -148,12 +149,34 @@ __host__ __device__ __forceinline__ int2 pair_slot(int N, int i, int j)
     const int a = i < j ? i : j, b = i < j ? j : i;
     return make_int2(a * (2 * N - a - 1) / 2 + (b - a - 1), i < j ? 0 : 1);
 }
-// index, in complex64 units, of element e of ADO q: paired ((plane * mp + q) * 2 + half)
-// or one plane per element (e * mp + q)
+// With N > kMaxStates the state is matrix-major, each matrix in panels of kWidePanel columns
+// (the last one narrower), row by row within a panel.  A 128-byte line then holds 2 x 4
+// elements in complex128 and 4 x 4 in complex64, and the row and the column of a state that
+// a bath mode couples to touch N / 4 lines and N / 2 (N / 4) of them, where plain rows would
+// touch N lines for the column alone.
+//   wide_pos: the position of element (i, j) in its matrix; wide_element: the inverse
+constexpr int kWidePanel = 4;
+__host__ __device__ __forceinline__ int wide_pos(int N, int i, int j)
+{
+    const int p = j / kWidePanel, w = N - p * kWidePanel < kWidePanel ? N - p * kWidePanel : kWidePanel;
+    return p * kWidePanel * N + i * w + (j - p * kWidePanel);
+}
+__host__ __device__ __forceinline__ int2 wide_element(int N, int pos)
+{
+    const int p = pos / (kWidePanel * N), r = pos - p * kWidePanel * N;
+    const int w = N - p * kWidePanel < kWidePanel ? N - p * kWidePanel : kWidePanel;
+    return make_int2(r / w, p * kWidePanel + r % w);
+}
+// Index of element e of ADO q in the state: one plane per element (e * mp + q), or matrix-major
+__host__ __device__ __forceinline__ int64_t state_index(int N, int e, int64_t q, int64_t mp)
+{
+    return N > kMaxStates ? q * (N * N) + wide_pos(N, e / N, e % N) : (int64_t)e * mp + q;
+}
+// the same in complex64 units, also for paired planes ((plane * mp + q) * 2 + half)
 __host__ __device__ __forceinline__ int64_t c64_index(bool paired, int N, int e, int64_t q, int64_t mp)
 {
     if (!paired)
-        return (int64_t)e * mp + q;
+        return state_index(N, e, q, mp);
     const int2 s = pair_slot(N, e / N, e % N);
     return ((int64_t)s.x * mp + q) * 2 + s.y;
 }
@@ -334,15 +357,43 @@ void launch_stage_adjoint(int N, int nterm_slots, bool real_h, int stage, const 
 
 // ---- large systems (stage_wide.hip): 8 < N <= 32, one wavefront per ADO ---------------
 
-// W: bath modes (the workgroup keeps its tile's slice of the neighbour table in LDS)
+// LDS row stride (complex elements) of one N x N matrix: odd, so that the 16 rows a matrix
+// core operand reads at once fall into different banks, and one of three, so that the places
+// of a lane's elements are constants of the kernels
+__host__ __device__ constexpr int wide_pitch(int N) { return N <= 16 ? 17 : N <= 24 ? 25 : 33; }
+// The neighbour terms by mode: mode m of class c couples the elements of the terms from
+// (c * W + m) * len on, at most len of them.  `where` holds for each the element's position in
+// the state (wide_pos, low half) and its place in a matrix of row stride wide_pitch(N) (high
+// half; 0xffff in the unused entries).  tile_order: the tiles with plus neighbours, then the
+// others.
+template <typename R>
+struct WideTables {
+    const TermT<R>* __restrict__ terms;
+    const uint32_t* __restrict__ where;
+    const int32_t* __restrict__ tile_order;
+    const uint16_t* __restrict__ place;  // [N*N] the LDS place of every position
+    int32_t W, len;
+};
+// the constants of the thermal state search (tss.hip): C and (i / hbar)(E_i - E_j) per
+// instance, eps - S_u and the uid (< 0: padding, kept at zero) per slot
+struct WideTss {
+    const double2* __restrict__ c;
+    const double2* __restrict__ w;
+    const double2* __restrict__ epsm;
+    const int32_t* __restrict__ q2u;
+};
+// W: bath modes
 bool wide_supported(int N, int complex_bytes, int W);
-// the largest number of ADOs per workgroup (a power of two <= 8) whose tiles fit in LDS
+// the largest number of wavefronts (ADOs at a time) per workgroup, a power of two <= 8
 int wide_max_ados(int N, int complex_bytes, int W);
-// ados: ADOs per workgroup, 0 = wide_max_ados
-void launch_stage_wide(int N, int nterm_slots, bool real_h, int stage, const StageArgsT<double>& a,
-                       const ElementArgsT<double>& el, int ados, hipStream_t s);
-void launch_stage_wide(int N, int nterm_slots, bool real_h, int stage, const StageArgsT<float>& a,
-                       const ElementArgsT<float>& el, int ados, hipStream_t s);
+// ados: wavefronts per workgroup, 0 = the default
+void launch_stage_wide(int N, bool real_h, int stage, const StageArgsT<double>& a, const ElementArgsT<double>& el,
+                       const WideTables<double>& wt, int ados, hipStream_t s);
+void launch_stage_wide(int N, bool real_h, int stage, const StageArgsT<float>& a, const ElementArgsT<float>& el,
+                       const WideTables<float>& wt, int ados, hipStream_t s);
+// one iteration of the thermal state search, a.yin -> a.yout
+void launch_tss_wide(int N, bool real_c, const StageArgsT<double>& a, const double2* gam, const WideTables<double>& wt,
+                     const WideTss& ts, hipStream_t s);
 
 // ---- paired pipelined launcher (stage_pair.hip), complex64 state --------------------
 

@@ -69,6 +69,25 @@ __device__ __forceinline__ int64_t plane_index(bool paired, int N, int e, int64_
     return c64_index(sizeof(C) == sizeof(float2) && paired, N, e, q, mp);
 }
 
+// Matrix-major states (N > kMaxStates): a copy of whole matrices between the two orders,
+// one workgroup per slot q; TO_STATE: dst[q] = src[u(q)] (0 for a slot without an ADO),
+// otherwise dst[u(q)] = src[q]
+template <typename C, bool TO_STATE>
+__global__ void copy_matrices(const double2* __restrict__ uid_order, C* __restrict__ state,
+                              double2* __restrict__ uid_out, const int32_t* __restrict__ q2u, int N)
+{
+    const int64_t q = blockIdx.x;
+    const int32_t u = q2u[q];
+    const int nel = N * N;
+    for (int e = threadIdx.x; e < nel; e += blockDim.x) {
+        const int64_t at = q * nel + wide_pos(N, e / N, e % N);
+        if (TO_STATE)
+            state[at] = from_d2<C>(u >= 0 ? uid_order[(int64_t)u * nel + e] : make_double2(0.0, 0.0));
+        else if (u >= 0)
+            uid_out[(int64_t)u * nel + e] = to_d2(state[at]);
+    }
+}
+
 // dst[e, q] = src[u(q)][e]   (reference AoS -> internal SoA; padding -> 0)
 template <typename C>
 __global__ void aos_to_soa(const double2* __restrict__ src, C* __restrict__ dst, const int32_t* __restrict__ q2u,
@@ -232,6 +251,34 @@ __global__ __launch_bounds__(64 * kNormWaves) void hierarchy_norm_kernel(const V
         mask[u] = 0;
 }
 
+// the same for matrix-major states (N > kMaxStates): one wavefront per ADO, lane = element,
+// four ADOs to a workgroup
+template <typename C>
+__global__ __launch_bounds__(256) void hierarchy_norm_matrices(const C* __restrict__ state, int nel,
+                                                               const int32_t* __restrict__ q2u, int64_t mp,
+                                                               double threshold, double* __restrict__ norms,
+                                                               uint8_t* __restrict__ mask)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int32_t u = q < mp ? q2u[q] : -1;
+    if (u < 0)
+        return;
+    double acc = 0.0;
+    for (int e = lane; e < nel; e += 64) {
+        const double2 v = to_d2(state[q * nel + e]);
+        acc = fma(v.x, v.x, acc);
+        acc = fma(v.y, v.y, acc);
+    }
+    for (int off = 32; off > 0; off >>= 1)
+        acc += __shfl_xor(acc, off);
+    if (lane == 0) {
+        norms[u] = acc;
+        if (acc - threshold <= 0.0 && mask[u] != 2)
+            mask[u] = 0;
+    }
+}
+
 // Fold the uid-order mask into the packed neighbour table: an edge whose target is
 // masked reads the zero slot (heom_ode.cl drops such a term with its mask checks).
 __global__ void fold_mask(const int2* __restrict__ raw, int2* __restrict__ folded, const uint8_t* __restrict__ mask,
@@ -248,17 +295,20 @@ __global__ void fold_mask(const int2* __restrict__ raw, int2* __restrict__ folde
     folded[t] = make_int2((int32_t)(((uint32_t)pf << 6) | (uint32_t)n), mf);
 }
 
-// new planes from old ones: dst[e * mp_new + q'] = src[e * mp_old + n2o[q']] (n2o < 0: zero)
-__global__ void remap_planes(const double2* __restrict__ src, double2* __restrict__ dst,
-                             const int32_t* __restrict__ n2o, int64_t mp_old, int64_t mp_new, int nel)
+// a new layout's state from the old one's: element e of slot q' from slot n2o[q'] (< 0: zero)
+__global__ void remap_state(const double2* __restrict__ src, double2* __restrict__ dst,
+                            const int32_t* __restrict__ n2o, int64_t mp_old, int64_t mp_new, int N)
 {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int nel = N * N;
     if (t >= (int64_t)nel * mp_new)
         return;
-    const int e = (int)(t / mp_new);
-    const int64_t qn = t % mp_new;
+    // t runs along the new layout's memory
+    const bool matrices = N > kMaxStates;
+    const int e = (int)(matrices ? t % nel : t / mp_new);
+    const int64_t qn = matrices ? t / nel : t % mp_new;
     const int32_t qo = n2o[qn];
-    dst[t] = qo >= 0 ? src[(int64_t)e * mp_old + qo] : make_double2(0.0, 0.0);
+    dst[t] = qo >= 0 ? src[matrices ? (int64_t)qo * nel + e : (int64_t)e * mp_old + qo] : make_double2(0.0, 0.0);
 }
 
 // sigma_q <- Mx_k sigma_q for every ADO q of instance k: wave = row i, lane = ADO,
@@ -293,7 +343,8 @@ __global__ __launch_bounds__(64 * N) void mmult_left_kernel(C* __restrict__ y, c
         y[plane_index<C>(paired, N, i * N + j, q, mp)] = from_d2<C>(out[j]);
 }
 
-// mmult_left for N > 8, out of place: out[e][q] = sum_k mx_ik y[k*N+j][q], thread = (e, q)
+// mmult_left for N > 8, out of place, matrix-major: out_ij = sum_k mx_ik y_kj for
+// every slot, thread = (slot, position)
 template <typename C>
 __global__ void mmult_left_wide(const C* __restrict__ y, C* __restrict__ out, const double2* __restrict__ mx,
                                 const int32_t* __restrict__ tile_inst, int64_t mp, int N)
@@ -302,13 +353,13 @@ __global__ void mmult_left_wide(const C* __restrict__ y, C* __restrict__ out, co
     const int nel = N * N;
     if (t >= (int64_t)nel * mp)
         return;
-    const int e = (int)(t / mp);
-    const int64_t q = t % mp;
-    const int i = e / N, j = e % N;
-    const double2* m = mx + (tile_inst ? (int64_t)tile_inst[q / kTile] * nel : 0);
+    const int64_t q = t / nel;
+    const int2 ij = wide_element(N, (int)(t % nel));
+    const double2* m = mx + (tile_inst ? (int64_t)tile_inst[q / kTile] * nel : 0) + ij.x * N;
+    const C* yq = y + q * nel;
     double2 acc = make_double2(0.0, 0.0);
     for (int k = 0; k < N; ++k)
-        acc = cfma(m[i * N + k], to_d2(y[(int64_t)(k * N + j) * mp + q]), acc);
+        acc = cfma(m[k], to_d2(yq[wide_pos(N, k, ij.y)]), acc);
     out[t] = from_d2<C>(acc);
 }
 
@@ -369,8 +420,9 @@ struct TierArgs {
 // workgroups: with two terms per element the kernel is held to 64 VGPRs (the commutator
 // loop unrolled twice, not more), so that 8 wavefronts per SIMD are resident, not 4; with
 // more terms it takes the registers it needs (no spills).
-template <int STAGE, int NT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT <= 2 ? 8 : 1))) void tier_fixup(TierArgs a)
+template <int STAGE, int NT, int THREADS>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(NT <= 2 ? 8 : THREADS / 256))) void tier_fixup(
+    TierArgs a)
 {
     extern __shared__ double2 tier_lds[];  // [nel] sigma, [nel] H / hbar, then [W] edges
     const int N = a.N, nel = N * N, W = a.W;
@@ -384,9 +436,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT <= 2 ? 8
     const int64_t q = a.q[s];
     const double2* in = a.in64 + (int64_t)s * nel;
     const double2* hs = a.hs + (int64_t)a.inst[s] * nel;
-    for (int e = threadIdx.x; e < nel; e += blockDim.x) {
+    // a thread has one element: what it reads of its own does not wait for the edges
+    const int e = threadIdx.x;
+    const bool mine = e < nel;
+    const double2 S = a.pfss[s];
+    const int cls = a.inst_class ? a.inst_class[a.inst[s]] : 0;
+    const Term* terms = a.terms + ((int64_t)cls * nel + e) * NT;
+    int mode[NT];
+    double2 g = make_double2(0.0, 0.0);
+    if (mine) {
         sig[e] = in[e];
         H[e] = hs[e];
+        g = a.gam[(int64_t)cls * nel + e];
+#pragma unroll
+        for (int k = 0; k < NT; ++k)
+            mode[k] = terms[k].mode;
     }
     for (int m = threadIdx.x; m < W; m += blockDim.x) {
         const int2 v = a.nb[(int64_t)m * a.mp + q];
@@ -394,22 +458,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT <= 2 ? 8
         spn[m] = a.sp_nb[(int64_t)s * W + m];
     }
     __syncthreads();
-    const double2 S = a.pfss[s];
-    const int cls = a.inst_class ? a.inst_class[a.inst[s]] : 0;
-    const Term* terms = a.terms + (int64_t)cls * nel * NT;
-    const double2* gam = a.gam + (int64_t)cls * nel;
-    for (int e = threadIdx.x; e < nel; e += blockDim.x) {
+    if (mine) {
         const int i = e / N, j = e - i * N;
         double2 xp[NT], xm[NT];
         int nv[NT];
 #pragma unroll
         for (int k = 0; k < NT; ++k) {
-            const int mode = terms[e * NT + k].mode;
             xp[k] = xm[k] = make_double2(0.0, 0.0);
             nv[k] = 0;
-            if (mode < W) {
-                const int4 ed = edge[mode];
-                const int2 sn = spn[mode];
+            if (mode[k] < W) {
+                const int4 ed = edge[mode[k]];
+                const int2 sn = spn[mode[k]];
                 nv[k] = ed.z;
                 if (ed.x != a.zero)
                     xp[k] = sn.x >= 0 ? a.in64[(int64_t)sn.x * nel + e]
@@ -426,11 +485,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT <= 2 ? 8
             const double2 hik = H[i * N + k];
             cm = cfma(make_double2(-hik.x, -hik.y), sig[k * N + j], cm);
         }
-        const double2 g = gam[e];
         double2 f = cfma(make_double2(S.x + g.x, S.y + g.y), sig[e], make_double2(-cm.y, cm.x));
 #pragma unroll
         for (int k = 0; k < NT; ++k) {
-            const Term tm = terms[e * NT + k];
+            const Term tm = terms[k];
             const double cp = tm.plus_c * sqrt((double)(nv[k] + 1));
             const double sm = sqrt((double)nv[k]);
             f.x = fma(-cp, xp[k].y, f.x);
@@ -507,26 +565,9 @@ template <typename R>
 void launch_stage_r(heom_handle* h, int stage, const unsigned char* yin, unsigned char* yout, double c1, bool reverse,
                     const ElementArgsT<R>& el, const c2<R>* pfss)
 {
-    StageArgsT<R> a{};
-    a.yin = reinterpret_cast<const c2<R>*>(yin);
-    a.y0 = h->y.as<c2<R>>();
-    a.pbuf = h->pbuf.as<c2<R>>();
-    a.yout = reinterpret_cast<c2<R>*>(yout);
-    a.nb = h->nb.p;
-    a.pfss = pfss;
-    a.tile_inst = h->count > 1 ? h->tile_inst.p : nullptr;
-    a.tile_plus = h->tile_plus.p;
-    a.tile_class = h->uniform ? nullptr : h->tile_class.p;
-    a.mp = h->Mp;
-    a.ntiles = h->ntiles;
-    a.zero_slot = h->zero_slot;
-    a.table_units = (h->W + 2) / 2;
-    a.xcd_chunk = h->xcd_chunk;
-    a.reverse = reverse ? 1 : 0;
-    a.split = h->pipelined ? 1 : h->tile_split;
-    a.c1 = (R)c1;
+    const StageArgsT<R> a = stage_args<R>(h, yin, h->y.p, h->pbuf.p, yout, c1, reverse, pfss);
     if (h->N > kMaxStates) {
-        heom_hip::launch_stage_wide(h->N, h->term_slots, h->real_h, stage, a, el, h->wide_ados, h->stream);
+        heom_hip::launch_stage_wide(h->N, h->real_h, stage, a, el, h->wide_tables<R>(), h->wide_ados, h->stream);
     } else if (h->pipelined) {
         if constexpr (std::is_same<R, float>::value)
             heom_hip::launch_stage_pair(h->N, h->pair_slots, h->real_h, stage, a, el, h->pterms.p, h->pipe_wgs,
@@ -537,6 +578,12 @@ void launch_stage_r(heom_handle* h, int stage, const unsigned char* yin, unsigne
         heom_hip::launch_stage(h->N, h->term_slots, h->real_h, stage, a, el, h->stream);
     }
     HIPC(hipGetLastError());
+}
+
+StageArgsT<double> stage_args64(heom_handle* h, const void* yin, const void* y0, void* pbuf, void* yout, double c1,
+                                bool reverse)
+{
+    return stage_args<double>(h, yin, y0, pbuf, yout, c1, reverse, h->pfss.p);
 }
 
 void launch_stage_buffers(heom_handle* h, int stage, const void* yin, const void* y0, void* pbuf, void* yout,
@@ -557,7 +604,7 @@ void launch_stage_buffers(heom_handle* h, int stage, const void* yin, const void
         const StageArgsT<double> a = stage_args<double>(h, yin, y0, pbuf, yout, c1, reverse, h->pfss.p);
         const ElementArgsT<double> el{h->hs.p, h->gam.p, h->terms.p};
         if (h->N > kMaxStates)
-            heom_hip::launch_stage_wide(h->N, h->term_slots, h->real_h, stage, a, el, h->wide_ados, h->stream);
+            heom_hip::launch_stage_wide(h->N, h->real_h, stage, a, el, h->wide_tables<double>(), h->wide_ados, h->stream);
         else if (h->pipelined)
             heom_hip::launch_stage_pipelined(h->N, h->term_slots, h->real_h, stage, a, el, h->pipe_wgs, h->stream);
         else
@@ -567,16 +614,25 @@ void launch_stage_buffers(heom_handle* h, int stage, const void* yin, const void
     h->timing.rhs_launches += 1;
 }
 
-template <int NT>
+template <int NT, int THREADS>
 void tier_fixup_stage(int stage, dim3 grid, dim3 block, size_t lds, hipStream_t st, const TierArgs& a)
 {
     switch (stage) {
-    case 0: hipLaunchKernelGGL((tier_fixup<0, NT>), grid, block, lds, st, a); break;
-    case 1: hipLaunchKernelGGL((tier_fixup<1, NT>), grid, block, lds, st, a); break;
-    case 2: hipLaunchKernelGGL((tier_fixup<2, NT>), grid, block, lds, st, a); break;
-    case 3: hipLaunchKernelGGL((tier_fixup<3, NT>), grid, block, lds, st, a); break;
-    default: hipLaunchKernelGGL((tier_fixup<4, NT>), grid, block, lds, st, a); break;
+    case 0: hipLaunchKernelGGL((tier_fixup<0, NT, THREADS>), grid, block, lds, st, a); break;
+    case 1: hipLaunchKernelGGL((tier_fixup<1, NT, THREADS>), grid, block, lds, st, a); break;
+    case 2: hipLaunchKernelGGL((tier_fixup<2, NT, THREADS>), grid, block, lds, st, a); break;
+    case 3: hipLaunchKernelGGL((tier_fixup<3, NT, THREADS>), grid, block, lds, st, a); break;
+    default: hipLaunchKernelGGL((tier_fixup<4, NT, THREADS>), grid, block, lds, st, a); break;
     }
+}
+
+template <int NT>
+void tier_fixup_threads(int stage, dim3 grid, int threads, size_t lds, hipStream_t st, const TierArgs& a)
+{
+    if (threads <= 256)
+        tier_fixup_stage<NT, 256>(stage, grid, dim3(threads), lds, st, a);
+    else
+        tier_fixup_stage<NT, 1024>(stage, grid, dim3(threads), lds, st, a);
 }
 
 // the FP64 pass over the tier-0/1 ADOs after a complex64 stage kernel
@@ -609,13 +665,16 @@ void tier_fixup_launch(heom_handle* h, int stage, const unsigned char* yin, unsi
     a.nt = h->term_slots;
     a.zero = h->zero_slot;
     a.c1 = c1;
-    // one workgroup per tier-0/1 ADO, a wavefront for N <= 8
-    const dim3 grid(h->S), block(std::min(256, (h->nel + 63) / 64 * 64));
+    // one workgroup per tier-0/1 ADO, a wavefront for N <= 8, a thread per element up to
+    // N = 32: the pass is a chain of round trips, and 24 x 24 elements on 256 threads took
+    // three of them
+    const dim3 grid(h->S);
+    const int block = std::min(1024, (h->nel + 63) / 64 * 64);
     const size_t lds = 2 * (size_t)h->nel * sizeof(double2) + (size_t)h->W * (sizeof(int4) + sizeof(int2));
     switch (h->term_slots) {
-    case 2: tier_fixup_stage<2>(stage, grid, block, lds, h->stream, a); break;
-    case 4: tier_fixup_stage<4>(stage, grid, block, lds, h->stream, a); break;
-    default: tier_fixup_stage<8>(stage, grid, block, lds, h->stream, a); break;
+    case 2: tier_fixup_threads<2>(stage, grid, block, lds, h->stream, a); break;
+    case 4: tier_fixup_threads<4>(stage, grid, block, lds, h->stream, a); break;
+    default: tier_fixup_threads<8>(stage, grid, block, lds, h->stream, a); break;
     }
     HIPC(hipGetLastError());
 }
@@ -732,6 +791,15 @@ void build_tile_plus(heom_handle* h, const std::vector<int2>& nb)
             if ((int32_t)((uint32_t)nb[(size_t)m * h->Mp + q].x >> 6) != h->zero_slot)
                 f[(size_t)(q / kTile)] = 1;
     upload(h->tile_plus, f, h->stream);
+    if (h->N > kMaxStates) {
+        std::vector<int32_t> order;
+        for (int want = 1; want >= 0; --want)
+            for (int t = 0; t < h->ntiles; ++t)
+                if (f[(size_t)t] == want)
+                    order.push_back(t);
+        upload(h->tile_order, order, h->stream);
+        HIPC(hipStreamSynchronize(h->stream));
+    }
 }
 
 // H [count][N*N*2] in J -> H / hbar on the device
@@ -840,6 +908,50 @@ void build_pair_terms(heom_handle* h, const std::vector<std::vector<Term>>& per,
     upload(h->pterms, flat, h->stream);
 }
 
+// N > 8: the neighbour terms by mode (WideTables in heom_device.hpp)
+void build_wide_terms(heom_handle* h, const std::vector<std::vector<Term>>& per, int C)
+{
+    const int N = h->N, W = h->W, nel = N * N;
+    std::vector<std::vector<Term>> by_mode((size_t)C * W);
+    for (int cl = 0; cl < C; ++cl)
+        for (int e = 0; e < nel; ++e)
+            for (Term t : per[(size_t)cl * nel + e]) {
+                std::vector<Term>& out = by_mode[(size_t)cl * W + t.mode];
+                t.mode = e;
+                out.push_back(t);
+            }
+    size_t len = 1;
+    for (const auto& m : by_mode)
+        len = std::max(len, m.size());
+    h->wide_len = (int)len;
+    std::vector<Term> flat(by_mode.size() * len, Term{});
+    std::vector<uint32_t> where(flat.size(), 0xffff0000u);
+    for (size_t m = 0; m < by_mode.size(); ++m) {
+        std::copy(by_mode[m].begin(), by_mode[m].end(), flat.begin() + (std::ptrdiff_t)(m * len));
+        for (size_t k = 0; k < by_mode[m].size(); ++k) {
+            const int i = by_mode[m][k].mode / N, j = by_mode[m][k].mode % N;
+            where[m * len + k] = (uint32_t)wide_pos(N, i, j) | (uint32_t)(i * wide_pitch(N) + j) << 16;
+        }
+    }
+    std::vector<uint16_t> place((size_t)nel);
+    for (int i = 0; i < N; ++i)
+        for (int j = 0; j < N; ++j)
+            place[(size_t)wide_pos(N, i, j)] = (uint16_t)(i * wide_pitch(N) + j);
+    upload(h->wplace, place, h->stream);
+    upload(h->wwhere, where, h->stream);
+    if (h->fp32()) {
+        std::vector<TermT<float>> f32(flat.size());
+        for (size_t t = 0; t < flat.size(); ++t)
+            f32[t] = {make_float2((float)flat[t].minus_c.x, (float)flat[t].minus_c.y), (float)flat[t].plus_c,
+                      flat[t].mode, flat[t].info};
+        upload(h->wterms32, f32, h->stream);
+        HIPC(hipStreamSynchronize(h->stream));
+    } else {
+        upload(h->wterms, flat, h->stream);
+        HIPC(hipStreamSynchronize(h->stream));
+    }
+}
+
 void build_coefficients(heom_handle* h)
 {
     const int N = h->N, W = h->W, C = (int)h->classes.size();
@@ -895,6 +1007,8 @@ void build_coefficients(heom_handle* h)
     if (N <= kMaxStates ? !stage_supported(N, most) : most > 8)
         raise(HEOM_E_UNSUPPORTED, "more than 8 neighbour terms per matrix element");
     h->term_slots = stage_term_slots(most);
+    if (N > kMaxStates)
+        build_wide_terms(h, per, C);
     // pad every element's list; padding terms read table column W, which always
     // holds the zero slot
     std::vector<Term> flat((size_t)C * N * N * h->term_slots);
@@ -1317,9 +1431,15 @@ void upload_state(heom_handle* h, const double* state, unsigned char* dst)
     DevBuf<double2> stage;
     stage.alloc((size_t)h->M * h->nel);
     HIPC(hipMemcpyAsync(stage.p, state, stage.bytes(), hipMemcpyHostToDevice, h->stream));
+    const bool matrices = h->N > kMaxStates;
+    const dim3 mgrid((unsigned)h->Mp), mblock(256);
     if (h->fp32()) {
-        hipLaunchKernelGGL(aos_to_soa<float2>, dim3(blocks_for(h->Mp, 256)), dim3(256), 0, h->stream, stage.p,
-                           h->y.as<float2>(), h->q2u.p, h->Mp, h->N, h->paired);
+        if (matrices)
+            hipLaunchKernelGGL((copy_matrices<float2, true>), mgrid, mblock, 0, h->stream, stage.p,
+                               h->y.as<float2>(), nullptr, h->q2u.p, h->N);
+        else
+            hipLaunchKernelGGL(aos_to_soa<float2>, dim3(blocks_for(h->Mp, 256)), dim3(256), 0, h->stream, stage.p,
+                               h->y.as<float2>(), h->q2u.p, h->Mp, h->N, h->paired);
         std::vector<double2> rows((size_t)h->S * h->nel);
         for (int s = 0; s < h->S; ++s)
             std::memcpy(&rows[(size_t)s * h->nel], state + (size_t)h->sp_uid[s] * h->nel * 2,
@@ -1329,8 +1449,13 @@ void upload_state(heom_handle* h, const double* state, unsigned char* dst)
         HIPC(hipGetLastError());
         HIPC(hipStreamSynchronize(h->stream));
     } else {
-        hipLaunchKernelGGL(aos_to_soa<double2>, dim3(blocks_for(h->Mp, 256)), dim3(256), 0, h->stream, stage.p,
-                           reinterpret_cast<double2*>(dst ? dst : h->y.p), h->q2u.p, h->Mp, h->N, false);
+        double2* to = reinterpret_cast<double2*>(dst ? dst : h->y.p);
+        if (matrices)
+            hipLaunchKernelGGL((copy_matrices<double2, true>), mgrid, mblock, 0, h->stream, stage.p, to, nullptr,
+                               h->q2u.p, h->N);
+        else
+            hipLaunchKernelGGL(aos_to_soa<double2>, dim3(blocks_for(h->Mp, 256)), dim3(256), 0, h->stream, stage.p, to,
+                               h->q2u.p, h->Mp, h->N, false);
         HIPC(hipGetLastError());
         HIPC(hipStreamSynchronize(h->stream));
     }
@@ -1344,7 +1469,14 @@ void download_state(heom_handle* h, const unsigned char* src, const double2* row
     stage.alloc((size_t)h->M * h->nel);
     if (h->active < h->M)  // ADOs removed by heom_compact read back as zero
         HIPC(hipMemsetAsync(stage.p, 0, stage.bytes(), h->stream));
-    if (h->fp32())
+    const dim3 mgrid((unsigned)h->Mp), mblock(256);
+    if (h->N > kMaxStates && h->fp32())
+        hipLaunchKernelGGL((copy_matrices<float2, false>), mgrid, mblock, 0, h->stream, nullptr,
+                           reinterpret_cast<float2*>(const_cast<unsigned char*>(src)), stage.p, h->q2u.p, h->N);
+    else if (h->N > kMaxStates)
+        hipLaunchKernelGGL((copy_matrices<double2, false>), mgrid, mblock, 0, h->stream, nullptr,
+                           reinterpret_cast<double2*>(const_cast<unsigned char*>(src)), stage.p, h->q2u.p, h->N);
+    else if (h->fp32())
         hipLaunchKernelGGL(soa_to_aos<float2>, dim3(blocks_for(h->Mp, 256)), dim3(256), 0, h->stream,
                            reinterpret_cast<const float2*>(src), stage.p, h->q2u.p, h->Mp, h->N, h->paired);
     else
@@ -1814,7 +1946,14 @@ int heom_hierarchy_norm(heom_handle* h, double threshold, double* norms)
         if (h->active < h->M)  // ADOs removed by heom_compact have norm 0
             HIPC(hipMemsetAsync(h->norms.p, 0, h->norms.bytes(), h->stream));
         const dim3 grid((unsigned)(h->Mp / kTile)), block(64 * kNormWaves);
-        if (h->fp32() && h->paired)
+        const dim3 mgrid((unsigned)((h->Mp + 3) / 4));
+        if (h->N > kMaxStates && h->fp32())
+            hipLaunchKernelGGL(hierarchy_norm_matrices<float2>, mgrid, dim3(256), 0, h->stream, h->y.as<float2>(),
+                               h->nel, h->q2u.p, h->Mp, threshold, h->norms.p, h->mask.p);
+        else if (h->N > kMaxStates)
+            hipLaunchKernelGGL(hierarchy_norm_matrices<double2>, mgrid, dim3(256), 0, h->stream, h->y.as<double2>(),
+                               h->nel, h->q2u.p, h->Mp, threshold, h->norms.p, h->mask.p);
+        else if (h->fp32() && h->paired)
             hipLaunchKernelGGL(hierarchy_norm_kernel<float4>, grid, block, 0, h->stream, h->y.as<float4>(),
                                pair_planes(h->N), h->q2u.p, h->Mp, threshold, h->norms.p, h->mask.p);
         else if (h->fp32())
@@ -2108,6 +2247,7 @@ int heom_device_bytes(heom_handle* h, int64_t* bytes)
         if (!bytes)
             raise(HEOM_E_INVALID, "bytes is NULL");
         int64_t b = h->y.bytes() + h->pbuf.bytes() + h->ya.bytes() + h->yb.bytes();
+        b += h->wterms.bytes() + h->wterms32.bytes() + h->wwhere.bytes();
         for (auto* x : {&h->pfss, &h->hs, &h->gam, &h->mx, &h->small, &h->y64, &h->sa64, &h->sb64, &h->p64,
                         &h->sp_pfss, &h->sp_tmp})
             b += x->bytes();
@@ -2225,8 +2365,8 @@ int heom_compact(heom_handle* h, int64_t* active)
         upload(n2o_d, n2o, h->stream);
         DevBuf<unsigned char> y_new;
         y_new.alloc((size_t)nel * mp * sizeof(double2));
-        hipLaunchKernelGGL(remap_planes, dim3(blocks_for((int64_t)nel * mp, 256)), dim3(256), 0, h->stream,
-                           h->y.as<double2>(), y_new.as<double2>(), n2o_d.p, Mp, mp, nel);
+        hipLaunchKernelGGL(remap_state, dim3(blocks_for((int64_t)nel * mp, 256)), dim3(256), 0, h->stream,
+                           h->y.as<double2>(), y_new.as<double2>(), n2o_d.p, Mp, mp, h->N);
         HIPC(hipGetLastError());
         HIPC(hipStreamSynchronize(h->stream));
         std::swap(h->y.p, y_new.p);

@@ -1,14 +1,23 @@
-// stage_wide.hip -- the HEOM RHS with the fused RK4 stage epilogue for large systems,
-// 8 < N <= 32 states (dm-heom/cl/heom/heom_ode.cl:24-451 plus rk_weighted_add.cl:19-106),
-// complex128 / FP64 and complex64 / FP32.
+// stage_wide.hip -- the HEOM RHS with the fused RK4 stage epilogue, and the thermal state
+// search's iteration, for large systems, 8 < N <= 32 states (dm-heom/cl/heom/heom_ode.cl
+// :24-451 plus rk_weighted_add.cl:19-106; thermal_state_search.cl:10-52), complex128 / FP64
+// and complex64 / FP32.
 //
-// The stage kernels for N <= 8 put one ADO on each lane and a 64-ADO tile of N^2
-// elements in LDS; at N = 24 that tile would need 590 KB.  Here a workgroup owns a
-// tile of T consecutive ADOs (a power of two up to 8 such that H and T matrices fit
-// the 144 KB LDS budget -- the most that fit unless the autotuner chose fewer; T
-// divides the 64-ADO instance granularity), and works in the three phases described
-// at the kernel: the commutator per ADO wavefront from LDS, everything that touches
-// global memory plane by plane across the tile's consecutive ADOs.
+// The state is matrix-major for these systems (heom_device.hpp: element e of ADO q at
+// q * N * N + e), and one wavefront works on one ADO at a time:
+//   * every access to the state, the stage operand and the outputs moves whole cache lines
+//     of one matrix (lane = element);
+//   * which neighbours an ADO has, and which matrices they are, is uniform over the
+//     wavefront: it walks the edges that exist (seven of 48 on average in a 24-mode
+//     hierarchy of depth 4), and for each the elements that its mode couples to (the rows
+//     and columns of its bath's states, 47 of 576 at one state per bath) as lanes;
+//   * the matrix goes to LDS once; the matrix cores take sigma H - H sigma from there as
+//     16 x 16 x 4 products (rows and columns beyond N are padding), and the result replaces
+//     the matrix in LDS, where the neighbour terms are added.
+// The wavefronts of a workgroup share only H / hbar and the "same" constants in LDS, so there
+// is a barrier only where the instance changes; the LDS accesses of one wavefront complete
+// in order.
+#include <algorithm>
 #include <type_traits>
 
 #include "heom_device.hpp"
@@ -18,291 +27,870 @@ namespace heom_hip {
 namespace {
 
 constexpr int kWideLdsBytes = 147456;  // 144 KB of the 160 KB LDS
-// a second instance with 48 KB, chosen when H and the tile fit: then up to three
-// workgroups share a CU instead of one, as far as their registers allow
-constexpr int kWideLdsSmallBytes = 49152;
+constexpr int kWideLdsAll = 163840;
 constexpr int kMaxWideStates = 32;
-
-// LDS row stride (complex elements) of one N x N matrix: one pad element breaks the
-// bank pattern of the 8 rows a wavefront reads at once
-__host__ __device__ constexpr int wide_row(int N) { return N + 1; }
-
-// at most 8 wavefronts per workgroup, so that a lane may hold up to 256 VGPRs (the
-// block's accumulators, operands and in-flight loads)
+// at most 8 wavefronts per workgroup, so that a lane may hold up to 256 VGPRs
 constexpr int kWideThreads = 512;
+// wavefronts on a SIMD (so on a CU four times as many, with which the grid walks the
+// hierarchy): as many as the registers of the kernel without spills allow (24 sites, 20,475
+// ADOs, ms per RK4 step: complex128 1.42 at 3 against 0.84 at 2, with the spills of 168
+// registers; complex64 0.57 at 4 against 0.54 at 3)
+template <typename R, int SZ>
+constexpr int kWideOccupancy = SZ <= 16                                 ? (sizeof(R) == sizeof(float) ? 5 : 4)
+                               : sizeof(R) == sizeof(float) && SZ <= 24 ? 3
+                                                                        : 2;
+constexpr int kWideCus = 256;
+// bytes of the places by mode that a workgroup keeps in LDS, at most
+constexpr int kWideWhereBytes = 16384;
+// modes whose neighbour loads are in flight together: more where a wavefront has one ADO at
+// most (ONE: no registers for the next one's matrix, and the ADOs with an edge in every mode
+// are the launch's critical path).  A mode costs its wavefront some 400 cycles of issue
+// besides the loads, so more of them ahead only wait for one another (ms per RK4 step at 24
+// sites, 20,475 ADOs: 0.682 with 2, 0.692 with 3, 0.728 with 4; at 9 sites, 715 ADOs, one
+// each: 0.0304 with 3, 0.0337 with 4).
+template <typename R, int SZ, bool ONE>
+constexpr int kWideModesAhead = SZ > 24 && sizeof(R) == sizeof(double) ? (ONE ? 2 : 1) : (ONE ? 3 : 2);
 
-// (ADO, element) pairs a thread carries through one pass of phase C
-constexpr int kWidePairsPerPass = 2;
-
-// table rows a workgroup copies to LDS for W modes: rows 0..W (mode W is the zero row
-// that padding terms name), rounded up to an even count
-__host__ __device__ constexpr int wide_table_rows(int W) { return (W + 2) & ~1; }
-
-// LDS bytes of a workgroup of T ADOs: H, the tile (later overwritten by the commutator-
-// plus-same-term values) and the tile's slice of the neighbour table
-__host__ __device__ constexpr int wide_lds_bytes(int N, int cbytes, int W, int T)
+// the size limit of the large-system kernels (a matrix of H and T more in kWideLdsBytes,
+// with the tile's slice of the neighbour table): what a handle may ask for
+__host__ __device__ constexpr int wide_limit_bytes(int N, int cbytes, int W, int T)
 {
-    return (T + 1) * N * wide_row(N) * cbytes + wide_table_rows(W) * T * (int)sizeof(int2);
+    return (T + 1) * N * (N + 1) * cbytes + ((W + 2) & ~1) * T * (int)sizeof(int2);
 }
 
-// ADOs per workgroup for N states with `cbytes` per complex element and W modes, 0 if
-// none fits
 int wide_tile(int N, int cbytes, int W)
 {
     for (int T = kWideThreads / 64; T >= 1; T /= 2)
-        if (wide_lds_bytes(N, cbytes, W, T) <= kWideLdsBytes)
+        if (wide_limit_bytes(N, cbytes, W, T) <= kWideLdsBytes)
             return T;
     return 0;
 }
 
-// Three phases per workgroup (T ADOs):
-//   A  the tile sigma and H / hbar into LDS, plane by plane (T consecutive ADOs of one
-//      element per T consecutive threads);
-//   B  wavefront = ADO: lane l owns the B x B block of elements (i, j) with
-//      i = (l / 8) * B + r, j = (l % 8) * B + c (B = ceil(N / 8)); the commutator of the
-//      block needs B rows of sigma and H and B columns of both per k, 4B LDS reads for
-//      B^2 complex products; after a barrier, commutator plus same term overwrite the
-//      tile in LDS;
-//   C  back to the plane-by-plane mapping: each thread takes (ADO, element) pairs, adds
-//      the element's neighbour terms (table entry and gathers) to the LDS value and runs
-//      the RK4 epilogue with the own element re-read from global memory (still in L2),
-//      so that loads of the stage operand and all stores move T consecutive ADOs of
-//      one plane together.  LDS: H and one tile, so that several workgroups share a CU.
-template <typename R, int B, int NT, int STAGE, bool REALH, int LDSB, int PP = kWidePairsPerPass>
-__global__ __launch_bounds__(kWideThreads) void rk4_stage_wide(StageArgsT<R> a, const c2<R>* __restrict__ hs_all,
-                                                               const c2<R>* __restrict__ gam,
-                                                               const TermT<R>* __restrict__ terms, int N, int T)
+// LDS of a workgroup of T wavefronts, in bytes: the constant matrix (H / hbar or C, complex or
+// its real part), the places by mode (where they take at most kWideWhereBytes), the "same"
+// constants (not beside 32 x 32 matrices in complex128), and a matrix per wavefront.  What lies
+// where is known at compile time: a pointer into either memory would make every access wait
+// for all loads under way.
+template <typename R, int SZ>
+constexpr bool kWideGamLds = sizeof(R) == sizeof(float) || SZ <= 24;
+struct WideLds {
+    int gam, where, mat, total;
+};
+__host__ __device__ constexpr int wide_round16(int b) { return (b + 15) / 16 * 16; }
+__host__ __device__ constexpr WideLds wide_lds(int N, int cbytes, bool real, bool gam_lds, int T, int where_bytes)
+{
+    const int m = N * wide_pitch(N), h = wide_round16((real ? cbytes / 2 : cbytes) * m), g = gam_lds ? cbytes * m : 0;
+    const int el = wide_round16(where_bytes);
+    return {h, h + g, h + g + el, h + g + el + T * cbytes * m};
+}
+// bytes of the places by mode in LDS, 0 if they stay in global memory
+int wide_where_bytes(int W, int len)
+{
+    const int64_t b = (int64_t)W * len * 4;
+    return b <= kWideWhereBytes ? (int)b : 0;
+}
+
+template <typename R>
+using v4 = R __attribute__((ext_vector_type(4)));
+
+// d += a b, 16 x 16 x 4: lane l holds a[l % 16][l / 16], b[l / 16][l % 16] and, in d, four
+// elements of column l % 16 at the rows d_row(l, 0..3)
+__device__ __forceinline__ v4<double> mfma(double a, double b, v4<double> c)
+{
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ v4<float> mfma(float a, float b, v4<float> c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+template <typename R>
+__device__ __forceinline__ int d_row(int lane, int v);
+template <>
+__device__ __forceinline__ int d_row<double>(int lane, int v)
+{
+    return (lane >> 4) + 4 * v;
+}
+template <>
+__device__ __forceinline__ int d_row<float>(int lane, int v)
+{
+    return 4 * (lane >> 4) + v;
+}
+
+// what one lane wrote to LDS before is what another lane of the wavefront reads after: the
+// hardware keeps a wavefront's LDS accesses in order, the compiler has to as well
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <typename R, int NB>
+struct Product {
+    v4<R> re[NB][NB], im[NB][NB];
+    __device__ __forceinline__ void clear()
+    {
+#pragma unroll
+        for (int a = 0; a < NB; ++a)
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+                re[a][b] = im[a][b] = v4<R>{R(0), R(0), R(0), R(0)};
+    }
+};
+
+// p += sigma M (LEFT = false) or M sigma, or with NEG minus that, M (real or complex) or its
+// transpose in LDS.  k = 4 s + l / 16 at step s; zero in k beyond N; rows and columns of the
+// result beyond N are not kept, so their operands may be anything inside the matrix.
+template <bool LEFT, bool TRANS, bool NEG, typename R, int NB, int NP, typename TM>
+__device__ __forceinline__ void multiply(Product<R, NB>& p, const c2<R>* sig, const TM* m, int N, int lane)
+{
+    constexpr bool REAL = sizeof(TM) == sizeof(R);
+    const int g = lane >> 4;
+    const c2<R>* xs[NB];
+    const TM* ys[NB];
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+        const int r = min(16 * t + (lane & 15), N - 1);
+        xs[t] = sig + (LEFT ? g * NP + r : r * NP + g);
+        ys[t] = m + (LEFT != TRANS ? r * NP + g : g * NP + r);
+    }
+    constexpr int XK = LEFT ? NP : 1, YK = LEFT != TRANS ? 1 : NP;  // strides in k
+    auto step = [&](int k0, bool in) {
+        c2<R> x[NB];
+        TM y[NB];
+#pragma unroll
+        for (int t = 0; t < NB; ++t) {
+            x[t] = xs[t][in ? k0 * XK : 0];
+            y[t] = ys[t][in ? k0 * YK : 0];
+            if (!in)
+                x[t] = mk2<R>(R(0), R(0));
+            if constexpr (REAL)
+                y[t] = in ? (NEG ? -y[t] : y[t]) : R(0);
+            else
+                y[t] = in ? (NEG ? mk2<R>(-y[t].x, -y[t].y) : y[t]) : mk2<R>(R(0), R(0));
+        }
+        auto add = [&](v4<R>& c, R xv, R yv) { c = LEFT ? mfma(yv, xv, c) : mfma(xv, yv, c); };
+#pragma unroll
+        for (int a = 0; a < NB; ++a)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const c2<R> xv = LEFT ? x[b] : x[a];
+                const TM yv = LEFT ? y[a] : y[b];
+                if constexpr (REAL) {
+                    add(p.re[a][b], xv.x, yv);
+                    add(p.im[a][b], xv.y, yv);
+                } else {
+                    add(p.re[a][b], xv.x, yv.x);
+                    add(p.re[a][b], -xv.y, yv.y);
+                    add(p.im[a][b], xv.y, yv.x);
+                    add(p.im[a][b], xv.x, yv.y);
+                }
+            }
+    };
+    int k0 = 0;
+#pragma unroll 2
+    for (; k0 + 4 <= N; k0 += 4)
+        step(k0, true);
+    if (k0 < N)
+        step(k0, k0 + g < N);
+}
+
+// p += sigma H - H sigma, complex128: the two products one after the other
+template <int NB, int NP, typename TM>
+__device__ __forceinline__ void commutator(Product<double, NB>& p, const double2* sig, const TM* h, int N, int lane)
+{
+    multiply<false, false, false, double, NB, NP>(p, sig, h, N, lane);
+    multiply<true, false, true, double, NB, NP>(p, sig, h, N, lane);
+}
+
+// The same for complex64, where the order of the sum shows in the sixth digit of small
+// elements: the products interleave in the k steps of the matrix cores, lane group
+// g = lane / 16 holding a factor of
+//   real H:     -H_ik sigma_kj (g = 0, 2) and sigma_ik H_kj (g = 1, 3), two k to a step;
+//   complex H:  sigma_ik H_kj as x.x, y.y and -H_ik sigma_kj as x.x, y.y (real part; the
+//               imaginary part x.y, y.x of each), one k to a step,
+// which sums every element in the order of k, as the scalar loop of the kernels for N <= 8
+// does.  A lane needs one element of sigma and one of H per step and 16-block: it is the left
+// operand of one product and the right operand of the other.
+template <int NB, int NP>
+__device__ __forceinline__ void commutator(Product<float, NB>& p, const float2* sig, const float* h, int N, int lane)
+{
+    const int g = lane >> 4;
+    const bool odd = g & 1;
+    const int xk = odd ? 1 : NP, hk = odd ? NP : 1;  // strides in k
+    const float2* xs[NB];
+    const float* ys[NB];
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+        const int r = min(16 * t + (lane & 15), N - 1), k = g >> 1;
+        xs[t] = sig + (odd ? r * NP + k : k * NP + r);
+        ys[t] = h + (odd ? k * NP + r : r * NP + k);
+    }
+    auto step = [&](int k0, bool in) {
+        float2 x[NB];
+        float y[NB];
+#pragma unroll
+        for (int t = 0; t < NB; ++t) {
+            x[t] = xs[t][in ? k0 * xk : 0];
+            y[t] = ys[t][in ? k0 * hk : 0];
+            if (!in)
+                x[t] = make_float2(0.f, 0.f);
+            y[t] = in ? (odd ? y[t] : -y[t]) : 0.f;
+        }
+#pragma unroll
+        for (int a = 0; a < NB; ++a)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                p.re[a][b] = mfma(odd ? x[a].x : y[a], odd ? y[b] : x[b].x, p.re[a][b]);
+                p.im[a][b] = mfma(odd ? x[a].y : y[a], odd ? y[b] : x[b].y, p.im[a][b]);
+            }
+    };
+    int k0 = 0;
+#pragma unroll 2
+    for (; k0 + 2 <= N; k0 += 2)
+        step(k0, true);
+    if (k0 < N)
+        step(k0, g < 2);
+}
+template <int NB, int NP>
+__device__ __forceinline__ void commutator(Product<float, NB>& p, const float2* sig, const float2* h, int N, int lane)
+{
+    const int g = lane >> 4;
+    const bool odd = g & 1, first = g < 2;  // first: sigma H
+    const int xk = first ? 1 : NP, hk = first ? NP : 1;
+    const float2 *xs[NB], *ys[NB];
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+        const int r = min(16 * t + (lane & 15), N - 1);
+        xs[t] = sig + (first ? r * NP : r);
+        ys[t] = h + (first ? r : r * NP);
+    }
+#pragma unroll 2
+    for (int k = 0; k < N; ++k) {
+        float2 x[NB], y[NB];
+#pragma unroll
+        for (int t = 0; t < NB; ++t) {
+            x[t] = xs[t][k * xk];
+            y[t] = ys[t][k * hk];
+        }
+#pragma unroll
+        for (int a = 0; a < NB; ++a)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                // left and right factors: re  (x.x, y.x), (-x.y, y.y) | (-y.x, x.x), (y.y, x.y)
+                //                         im  (x.x, y.y), (x.y, y.x)  | (-y.x, x.y), (-y.y, x.x)
+                const float ar = first ? (odd ? -x[a].y : x[a].x) : (odd ? y[a].y : -y[a].x);
+                const float br = first ? (odd ? y[b].y : y[b].x) : (odd ? x[b].y : x[b].x);
+                const float ai = first ? (odd ? x[a].y : x[a].x) : (odd ? -y[a].y : -y[a].x);
+                const float bi = first ? (odd ? y[b].x : y[b].y) : (odd ? x[b].x : x[b].y);
+                p.re[a][b] = mfma(ar, br, p.re[a][b]);
+                p.im[a][b] = mfma(ai, bi, p.im[a][b]);
+            }
+    }
+}
+
+// value = fn(place, i, j, value) for the elements (i, j) of a product that lie in N x N;
+// place = i * NP + j
+template <typename R, int NB, int NP, typename Fn>
+__device__ __forceinline__ void each_element(Product<R, NB>& p, int N, int lane, Fn&& fn)
+{
+    const int i0 = d_row<R>(lane, 0), j0 = lane & 15, at0 = i0 * NP + j0;
+#pragma unroll
+    for (int a = 0; a < NB; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int di = 16 * a + d_row<R>(0, v), dj = 16 * b;
+                if (i0 + di < N && j0 + dj < N) {
+                    const c2<R> r = fn(at0 + di * NP + dj, i0 + di, j0 + dj, mk2<R>(p.re[a][b][v], p.im[a][b][v]));
+                    p.re[a][b][v] = r.x;
+                    p.im[a][b][v] = r.y;
+                }
+            }
+}
+
+// the value of `tab` in lane `idx`, the same in every lane
+__device__ __forceinline__ double uniform_lane(double tab, int idx)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(tab), idx),
+                            __builtin_amdgcn_readlane(__double2loint(tab), idx));
+}
+__device__ __forceinline__ float uniform_lane(float tab, int idx)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tab), idx));
+}
+
+// one ADO's lanes of 64 modes' table entries
+struct EdgeLanes {
+    int2 v;
+    __device__ __forceinline__ void load(const int2* nb, int64_t mp, int64_t q, int m, int W, int zero_slot)
+    {
+        v = m < W ? nb[(int64_t)m * mp + q] : make_int2((int32_t)((uint32_t)zero_slot << 6), zero_slot);
+    }
+};
+
+// The neighbour terms of one ADO, summed into the matrix f in LDS: for every element in the
+// order of the modes, plus before minus.  Its edges in modes m0 .. m0 + 63 are in the lanes of
+// `ed`; the modes with an edge are walked with D of them in flight (a mode that couples to
+// more than 64 elements counts as several).  Every mode makes the same loads -- through a
+// buffer resource that ends at once where the edge is missing, so that nothing is read and
+// zeros come back -- and so the wait for one mode's loads is not one for those behind it.
+// `where` is this class's, in LDS where it fits.
+template <typename R, int D>
+struct Neighbours {
+    using C = c2<R>;
+    using V = vec2_t<R>;
+    const StageArgsT<R>& a;
+    const WideTables<R>& wt;
+    const TermT<R>* terms;
+    const uint32_t* where;
+    int64_t q;
+    int nel, lane, m0 = 0, chunk = 0, todo;
+    EdgeLanes ed;
+    uint64_t has_p, has_m, left;
+    V mc[D], xp[D], xm[D];
+    R pc[D];
+    int at[D], n[D];
+
+    __device__ __forceinline__ Neighbours(const StageArgsT<R>& a_, const WideTables<R>& wt_, int cls,
+                                          const uint32_t* where_, EdgeLanes entries, int64_t q_, int nel_, int lane_)
+        : a(a_), wt(wt_), terms(wt_.terms + (int64_t)cls * wt_.W * wt_.len), where(where_), q(q_), nel(nel_),
+          lane(lane_), ed(entries)
+    {
+        begin();
+    }
+    __device__ __forceinline__ void begin()
+    {
+        has_p = __ballot((int32_t)((uint32_t)ed.v.x >> 6) != a.zero_slot);
+        has_m = __ballot(ed.v.y != a.zero_slot);
+        left = has_p | has_m;
+        todo = __popcll(left) * ((wt.len + 63) / 64);
+        chunk = 0;
+#pragma unroll
+        for (int u = 0; u < D; ++u)
+            fetch(u);
+    }
+    __device__ __forceinline__ V element(int64_t slot, bool there, int pos) const
+    {
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(a.yin + slot * nel), (short)0, there ? nel * (int)sizeof(C) : 0, 0x00020000);
+        if constexpr (sizeof(C) == 16) {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, pos * (int)sizeof(C), 0, 0);
+            return V{__hiloint2double((int)v[1], (int)v[0]), __hiloint2double((int)v[3], (int)v[2])};
+        } else {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, pos * (int)sizeof(C), 0, 0);
+            return V{__int_as_float((int)v[0]), __int_as_float((int)v[1])};
+        }
+    }
+    // requests the next mode (none left: loads that read nothing, or a term that is not used)
+    __device__ __forceinline__ void fetch(int u)
+    {
+        const bool some = left != 0;
+        const int m = some ? __builtin_ctzll(left) : 0;
+        const int vx = __builtin_amdgcn_readlane(ed.v.x, m), vy = __builtin_amdgcn_readlane(ed.v.y, m);
+        const int k = chunk * 64 + lane, i = (m0 + m) * wt.len + min(k, wt.len - 1);
+        const uint32_t pp = where[i];
+        const bool p = (has_p >> m & 1) && some, mn = (has_m >> m & 1) && some;
+        xp[u] = element(p ? (int64_t)((uint32_t)vx >> 6) : 0, p, (int)(pp & 0xffff));
+        xm[u] = element(mn ? (int64_t)(uint32_t)vy : 0, mn, (int)(pp & 0xffff));
+        mc[u] = V{terms[i].minus_c.x, terms[i].minus_c.y};
+        pc[u] = terms[i].plus_c;
+        at[u] = some && k < wt.len ? (int)(pp >> 16) : 0xffff;
+        n[u] = vx & 63;
+        if (++chunk * 64 >= wt.len) {
+            chunk = 0;
+            left &= left - 1;
+        }
+    }
+    template <bool SCALED>
+    __device__ __forceinline__ void add(int u, R scale, R sq_lane, C* f)
+    {
+        const R sp = uniform_lane(sq_lane, n[u] + 1), sm = uniform_lane(sq_lane, n[u]);
+        const R cp = SCALED ? scale * (pc[u] * sp) : pc[u] * sp, cm = SCALED ? scale * sm : sm;
+        if (at[u] != 0xffff) {
+            C s = f[at[u]];
+            s.x = fma(-cp, xp[u].y, s.x);
+            s.y = fma(cp, xp[u].x, s.y);
+            f[at[u]] = cfma(mk2<R>(mc[u].x, mc[u].y), mk2<R>(cm * xm[u].x, cm * xm[u].y), s);
+        }
+        wave_sync();
+    }
+    template <bool SCALED>
+    __device__ __forceinline__ void run(R scale, R sq_lane, C* f)
+    {
+        for (;;) {
+            for (; todo > D; todo -= D)
+#pragma unroll
+                for (int u = 0; u < D; ++u) {
+                    add<SCALED>(u, scale, sq_lane, f);
+                    fetch(u);
+                }
+#pragma unroll
+            for (int u = 0; u < D; ++u)
+                if (u < todo)
+                    add<SCALED>(u, scale, sq_lane, f);
+            m0 += 64;
+            if (m0 >= wt.W)
+                break;
+            ed.load(a.nb, a.mp, q, m0 + lane, wt.W, a.zero_slot);
+            begin();
+        }
+    }
+};
+
+// The sequence of groups of T consecutive ADOs (one per wavefront) of a workgroup: the tiles
+// in tile_order are dealt to the XCDs in turn, a tile's groups to the XCD's workgroups in
+// turn.  T divides the 64-ADO tile, so a group has one instance and one bath class.  The tiles
+// with plus neighbours come first in the order: their ADOs have several times the edges of the
+// others, and every workgroup gets its share of them.
+struct Walk {
+    const int32_t* order;
+    int x, j, gx, per, T, nt;
+    __device__ __forceinline__ Walk(const int32_t* order_, int ntiles, int T_)
+        : order(order_), x((int)(blockIdx.x % kNumXcd)), j((int)(blockIdx.x / kNumXcd)),
+          gx((int)(gridDim.x / kNumXcd)), per(kTile / T_), T(T_), nt(ntiles)
+    {
+    }
+    // the first ADO of the XCD's jj-th group, or -1 past the end (IN_ORDER: of the tiles as
+    // they lie, without a look at tile_order: where every workgroup has one group)
+    template <bool IN_ORDER>
+    __device__ __forceinline__ int64_t group(int jj) const
+    {
+        const int t = jj / per * kNumXcd + x;
+        if (t >= nt)
+            return -1;
+        return (int64_t)(IN_ORDER ? t : __builtin_amdgcn_readfirstlane(order[t])) * kTile + jj % per * T;
+    }
+};
+
+// one matrix in registers, lane = element: NL elements per lane
+template <typename R, int NL>
+struct Lin {
+    vec2_t<R> v[NL];
+    __device__ __forceinline__ c2<R> operator[](int k) const { return mk2<R>(v[k].x, v[k].y); }
+    __device__ __forceinline__ void load(const c2<R>* p, int nel, int lane)
+    {
+#pragma unroll
+        for (int k = 0; k < NL; ++k)
+            if (lane + 64 * k < nel)
+                v[k] = *reinterpret_cast<const vec2_t<R>*>(p + lane + 64 * k);
+    }
+    __device__ __forceinline__ void load_nt(const c2<R>* p, int nel, int lane)
+    {
+#pragma unroll
+        for (int k = 0; k < NL; ++k)
+            if (lane + 64 * k < nel)
+                v[k] = __builtin_nontemporal_load(reinterpret_cast<const vec2_t<R>*>(p + lane + 64 * k));
+    }
+};
+
+// the workgroup's constants in LDS: M (H / hbar or C; its real part for TM = R), gam and the
+// places by mode
+template <typename R, typename TM, int SZ, bool WLDS>
+__device__ __forceinline__ void load_constants(const c2<R>* __restrict__ m, const c2<R>* __restrict__ gam,
+                                               const uint32_t* __restrict__ where, int terms, int N, TM* ml,
+                                               c2<R>* gl, uint32_t* el, bool first)
+{
+    const int NP = wide_pitch(N);
+    const uint32_t ninv = (1u << 20) / (uint32_t)N + 1u;
+    if (!first)
+        __syncthreads();  // nobody uses the previous ones any more
+    // the loads of up to four rounds before the first store
+    constexpr int U = SZ <= 16 ? 1 : 4;
+    constexpr bool GL = kWideGamLds<R, SZ>;
+    const int n = N * N, step = (int)blockDim.x;
+    for (int e0 = threadIdx.x; e0 < n; e0 += U * step) {
+        vec2_t<R> mv[U], gv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e = min(e0 + u * step, n - 1);
+            mv[u] = vec2_t<R>{m[e].x, m[e].y};
+            if (GL)
+                gv[u] = vec2_t<R>{gam[e].x, gam[e].y};
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e = min(e0 + u * step, n - 1);  // past the end: the last element again
+            const int at = e + (NP - N) * (int)(((uint32_t)e * ninv) >> 20);
+            if constexpr (sizeof(TM) == sizeof(R))
+                ml[at] = mv[u].x;
+            else
+                ml[at] = mk2<R>(mv[u].x, mv[u].y);
+            if (GL)
+                gl[at] = mk2<R>(gv[u].x, gv[u].y);
+        }
+    }
+    if (WLDS)
+        for (int i0 = threadIdx.x; i0 < terms; i0 += U * step) {
+            uint32_t v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                v[u] = where[min(i0 + u * step, terms - 1)];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                el[min(i0 + u * step, terms - 1)] = v[u];
+        }
+    __syncthreads();
+}
+
+// One RK4 stage (STAGE 1..4, or 0: the RHS alone) over the whole hierarchy.  N <= SZ.
+template <typename R, int SZ, int STAGE, bool REALH, bool ONE, bool WLDS>
+__global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(kWideOccupancy<R, SZ>)))
+void rk4_stage_wide(StageArgsT<R> a, WideTables<R> wt,
+                                                               const c2<R>* __restrict__ hs_all,
+                                                               const c2<R>* __restrict__ gam_all, int N_, int T)
 {
     using C = c2<R>;
-    __shared__ C lds[LDSB / sizeof(C)];
-    __shared__ R sqrt_n[64];  // sqrt(n), n = 0..63
-    const int nel = N * N, NP = wide_row(N), mat = N * NP;
-    C* hl = lds;         // [N][NP] H / hbar
-    C* sig = lds + mat;  // [T][N][NP] the tile, then commutator + same term
-    int2* tabl = reinterpret_cast<int2*>(sig + T * mat);  // [rows][T] the tile's table slice
-    const int trows = 2 * a.table_units;
-    // index arithmetic without runtime divisions: T is a power of two, and
-    // e / N = (e * ninv) >> 20 for every e < 8256 and N <= 32
-    const int tsh = __builtin_ctz((unsigned)T);
-    const uint32_t ninv = (1u << 20) / (uint32_t)N + 1u;
-    auto div_n = [&](int e) { return (int)(((uint32_t)e * ninv) >> 20); };
-
-    const int64_t mp = a.mp;
-    // XCD-aware order: runs of 16 consecutive workgroups (16 T ADOs) on one XCD
-    const int64_t q0 = (int64_t)xcd_tile(blockIdx.x, gridDim.x, 16) * T;
-    const C* hs = hs_all + (a.tile_inst ? (int64_t)a.tile_inst[q0 / kTile] * nel : 0);
-    const int cls = tile_bath_class(a, (int)(q0 / kTile));
-    gam += cls * nel;
-    terms += cls * nel * NT;
-    if (threadIdx.x < 64)
-        sqrt_n[threadIdx.x] = sqrt((R)threadIdx.x);
-    for (int idx = threadIdx.x; idx < nel; idx += blockDim.x) {
-        const int r = div_n(idx);
-        hl[r * NP + idx - r * N] = hs[idx];
+    using TM = std::conditional_t<REALH, R, C>;
+    constexpr int NB = (SZ + 15) / 16, NL = (SZ * SZ + 63) / 64, NP = wide_pitch(SZ);
+    // complex128: the neighbour terms are added, times c1, to the value that already holds
+    // the rest of the result; complex64: they are summed by themselves (stages 1 and 4),
+    // since one rounding more or less shows there
+    constexpr bool LINEAR = STAGE == 1 || STAGE == 4;
+    constexpr bool APART = LINEAR && sizeof(R) == sizeof(float);
+    // the next ADO's matrix goes to registers during the neighbour terms (36 at most; stage 2
+    // needs its own values to the end and loads the next ones after that)
+    constexpr bool EARLY = STAGE != 2 && NL * sizeof(C) <= 144;
+    extern __shared__ __align__(16) unsigned char wide_mem[];
+    // one round trip for the arguments that the first loads need, not one at each of them
+    if (ONE)
+        asm volatile("" ::"s"(a.yin), "s"(a.nb), "s"(a.mp), "s"(a.pfss), "s"(a.tile_inst), "s"(a.tile_class), "s"(wt.place),
+                     "s"(wt.where), "s"(wt.terms), "s"(wt.W), "s"(wt.len), "s"(hs_all), "s"(gam_all), "s"(N_), "s"(T),
+                     "s"(a.zero_slot), "s"(a.ntiles), "s"(a.y0), "s"(a.yout));
+    const int nel = N_ * N_;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int terms = wt.W * wt.len;
+    constexpr bool GL = kWideGamLds<R, SZ>;
+    const WideLds L = wide_lds(N_, (int)sizeof(C), REALH, GL, T, WLDS ? terms * 4 : 0);
+    TM* hl = reinterpret_cast<TM*>(wide_mem);
+    C* gl = reinterpret_cast<C*>(wide_mem + L.gam);
+    uint32_t* el = reinterpret_cast<uint32_t*>(wide_mem + L.where);
+    C* sig = reinterpret_cast<C*>(wide_mem + L.mat) + (int64_t)w * (N_ * NP);  // this wavefront's matrix
+    int places[(NL + 1) / 2];  // of this lane's elements, two to a register
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
+        const int at = wt.place[min((int)(threadIdx.x & 63) + 64 * k, nel - 1)];
+        places[k / 2] = k & 1 ? places[k / 2] | at << 16 : at;
     }
-    for (int idx = threadIdx.x; idx < T * nel; idx += blockDim.x) {
-        const int ad = idx & (T - 1), e = idx >> tsh, r = div_n(e);
-        sig[ad * mat + r * NP + e - r * N] = a.yin[(int64_t)e * mp + q0 + ad];
-    }
-    for (int idx = threadIdx.x; idx < trows * T; idx += blockDim.x)
-        tabl[idx] = a.nb[(int64_t)(idx >> tsh) * mp + q0 + (idx & (T - 1))];
-    __syncthreads();
+    auto place = [&](int k) { return k & 1 ? (int)((uint32_t)places[k / 2] >> 16) : places[k / 2] & 0xffff; };
+    const R sq_lane = sqrt((R)(threadIdx.x & 63));  // sqrt(n), n = 0..63, one value per lane
 
-    // phase B
-    {
-        const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        const int lane = threadIdx.x & 63;
-        const int i0 = (lane >> 3) * B, j0 = (lane & 7) * B;
-        const C S = a.pfss[q0 + wv];
-        const C* s = sig + wv * mat;
-        int ir[B], jc[B];
-#pragma unroll
-        for (int r = 0; r < B; ++r) {
-            ir[r] = i0 + r < N ? i0 + r : 0;  // rows beyond N read row 0 and are not kept
-            jc[r] = j0 + r < N ? j0 + r : 0;
-        }
-        C cm[B][B];
-#pragma unroll
-        for (int r = 0; r < B; ++r)
-#pragma unroll
-            for (int c = 0; c < B; ++c)
-                cm[r][c] = mk2<R>(R(0), R(0));
-#pragma unroll 4
-        for (int k = 0; k < N; ++k) {
-            C sik[B], hik[B], hkj[B], skj[B];
-#pragma unroll
-            for (int r = 0; r < B; ++r) {
-                sik[r] = s[ir[r] * NP + k];
-                hik[r] = hl[ir[r] * NP + k];
-                hkj[r] = hl[k * NP + jc[r]];
-                skj[r] = s[k * NP + jc[r]];
+    const Walk walk(wt.tile_order, a.ntiles, T);
+    int j = walk.j, inst = -1, cls = -1;
+    const int lane_ = threadIdx.x & 63;
+    int64_t q0 = walk.template group<ONE>(j);
+    if (q0 < 0)
+        return;  // the whole workgroup leaves together
+    // a wavefront whose slot holds no ADO (the last tile's padding) goes through the motions
+    // with the last ADO and stores nothing
+    auto slot = [&](int64_t g) { return min(g + w, (int64_t)a.zero_slot - 1); };
+    Lin<R, NL> own;
+    EdgeLanes ed;
+    own.load(a.yin + slot(q0) * nel, nel, lane_);
+    ed.load(a.nb, a.mp, slot(q0), lane_, wt.W, a.zero_slot);
+    for (;;) {
+        const int it = a.tile_inst ? a.tile_inst[q0 / kTile] : 0;
+        const int cl = tile_bath_class(a, (int)(q0 / kTile));
+        const C* gam = gam_all + (int64_t)cl * nel;
+        const uint32_t* where = wt.where + (int64_t)cl * terms;
+        if (it != inst || cl != cls)
+            load_constants<R, TM, SZ, WLDS>(hs_all + (int64_t)it * nel, gam, where, terms, N_, hl, gl, el, inst < 0);
+        inst = it;
+        cls = cl;
+        j += walk.gx;
+        const int64_t q = slot(q0), q0n = ONE ? -1 : walk.template group<ONE>(j);
+        const bool live = q0 + w < a.zero_slot;
+        auto ahead = [&](bool edges, bool matrix) {  // the next ADO's
+            if (q0n >= 0) {
+                if (edges)
+                    ed.load(a.nb, a.mp, slot(q0n), lane_, wt.W, a.zero_slot);
+                if (matrix)
+                    own.load(a.yin + slot(q0n) * nel, nel, lane_);
             }
+        };
+        // the masks and addresses of the elements are formed where they are used: kept over
+        // the loop they would not fit the registers
+        int lane = lane_, N = N_;
+        asm volatile("" : "+v"(lane), "+s"(N));
+        const C S = a.pfss[q];
+        Lin<R, NL> ep;
+        auto operand = [&] {
+            if (STAGE == 2 || STAGE == 3)
+                ep.load_nt(a.y0 + q * nel, nel, lane);
+            if (STAGE == 4)
+                ep.load_nt(a.pbuf + q * nel, nel, lane);
+        };
+        {
 #pragma unroll
-            for (int r = 0; r < B; ++r)
-#pragma unroll
-                for (int c = 0; c < B; ++c) {
-                    if (REALH) {
-                        cm[r][c].x = fma(sik[r].x, hkj[c].x, fma(-hik[r].x, skj[c].x, cm[r][c].x));
-                        cm[r][c].y = fma(sik[r].y, hkj[c].x, fma(-hik[r].x, skj[c].y, cm[r][c].y));
-                    } else {
-                        cm[r][c] = cfma(sik[r], hkj[c], cm[r][c]);
-                        cm[r][c] = cfma(mk2<R>(-hik[r].x, -hik[r].y), skj[c], cm[r][c]);
-                    }
-                }
-        }
-        C fv[B][B];
-#pragma unroll
-        for (int r = 0; r < B; ++r)
-#pragma unroll
-            for (int c = 0; c < B; ++c) {
-                const int i = ir[r], j = jc[c];
-                const C g = gam[i * N + j];
-                const C own = s[i * NP + j];
-                const C fb = cfma(mk2<R>(S.x + g.x, S.y + g.y), own, mk2<R>(-cm[r][c].y, cm[r][c].x));
+            for (int k = 0; k < NL; ++k)
+                if (lane + 64 * k < nel)
+                    sig[place(k)] = own[k];
+            wave_sync();
+            // the first neighbours are under way during the commutator
+            Neighbours<R, kWideModesAhead<R, SZ, ONE>> nbs(a, wt, cl, WLDS ? el : where, ed, q, nel, lane);
+            __builtin_amdgcn_sched_barrier(0);
+
+            Product<R, NB> cm;  // sigma H - H sigma (over hbar)
+            cm.clear();
+            commutator<NB, NP>(cm, sig, hl, N, lane);
+            wave_sync();
+            each_element<R, NB, NP>(cm, N, lane, [&](int at, int i, int jj, C c) {
+                const C g = GL ? gl[at] : gam[i * N + jj];
+                const C s = sig[at];
+                const C fb = cfma(mk2<R>(S.x + g.x, S.y + g.y), s, mk2<R>(-c.y, c.x));
                 // stages 1 and 4 take the element's own value linearly (s + c1 f, and
-                // (ep + s) / 3 + c1 f): its part goes into the LDS value here, so that
-                // phase C needs no second read of it
+                // (ep + s) / 3 + c1 f): its part goes in here
+                C r = fb;
                 if (STAGE == 1)
-                    fv[r][c] = mk2<R>(fma(a.c1, fb.x, own.x), fma(a.c1, fb.y, own.y));
+                    r = mk2<R>(fma(a.c1, fb.x, s.x), fma(a.c1, fb.y, s.y));
                 else if (STAGE == 4)
-                    fv[r][c] = mk2<R>(fma(own.x, R(1) / R(3), a.c1 * fb.x), fma(own.y, R(1) / R(3), a.c1 * fb.y));
-                else
-                    fv[r][c] = fb;
-            }
-        __syncthreads();  // every wavefront is done reading the tile
-        C* fo = sig + wv * mat;
-#pragma unroll
-        for (int r = 0; r < B; ++r)
-#pragma unroll
-            for (int c = 0; c < B; ++c)
-                if (i0 + r < N && j0 + c < N)
-                    fo[(i0 + r) * NP + j0 + c] = fv[r][c];
-    }
-    __syncthreads();
-
-    // phase C, PP (ADO, element) pairs per thread and pass so that their loads overlap
-    // (table entries from LDS, then the gathers, stage operands and own values together);
-    // PLUS = false (no ADO of the 64-ADO tile that holds these T has a plus neighbour)
-    // leaves out the plus gathers
-    auto phase_c = [&](auto plus_tag) {
-        constexpr bool PLUS = decltype(plus_tag)::value;
-        const int total = T * nel, stride = blockDim.x;
-        for (int base = threadIdx.x; base < total; base += PP * stride) {
-            int2 nbv[PP][NT];
-            C ep[PP], own[PP], xp[PP][NT], xm[PP][NT];
-            int64_t o[PP];
-            int e2[PP], lo[PP];
-            bool live[PP];
-#pragma unroll
-            for (int u = 0; u < PP; ++u) {
-                const int idx = base + u * stride;
-                live[u] = idx < total;
-                const int id = live[u] ? idx : base;  // a dead pair repeats the first pair's loads
-                const int ad = id & (T - 1), e = id >> tsh, r = div_n(e);
-                e2[u] = e;
-                lo[u] = ad * mat + r * NP + e - r * N;
-                o[u] = (int64_t)e * mp + q0 + ad;
-#pragma unroll
-                for (int k = 0; k < NT; ++k)
-                    nbv[u][k] = tabl[terms[e * NT + k].mode * T + ad];
-                ep[u] = stage_operand<STAGE, R>(a, o[u]);
-                if (STAGE == 2)  // stages 1 and 4 have it in the LDS value, 0 and 3 do not use it
-                    own[u] = a.yin[o[u]];
+                    r = mk2<R>(fma(s.x, R(1) / R(3), a.c1 * fb.x), fma(s.y, R(1) / R(3), a.c1 * fb.y));
+                sig[at] = APART ? mk2<R>(R(0), R(0)) : r;
+                return r;
+            });
+            wave_sync();
+            __builtin_amdgcn_sched_barrier(0);
+            operand();  // the neighbour terms cover it
+            nbs.template run<LINEAR && !APART>(a.c1, sq_lane, sig);
+            if (!ONE)
+                ahead(true, EARLY);
+            wave_sync();
+            if (APART) {
+                each_element<R, NB, NP>(cm, N, lane, [&](int at, int, int, C r) {
+                    const C f = sig[at];
+                    sig[at] = mk2<R>(fma(a.c1, f.x, r.x), fma(a.c1, f.y, r.y));
+                    return r;
+                });
+                wave_sync();
             }
 #pragma unroll
-            for (int u = 0; u < PP; ++u) {
-                const C* plane = a.yin + (int64_t)e2[u] * mp;
-#pragma unroll
-                for (int k = 0; k < NT; ++k) {
-                    if constexpr (PLUS)
-                        xp[u][k] = plane[(uint32_t)nbv[u][k].x >> 6];
-                    xm[u][k] = plane[(uint32_t)nbv[u][k].y];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < PP; ++u) {
-                if (!live[u])
+            for (int k = 0; k < NL; ++k) {
+                const int e = lane + 64 * k;  // position
+                if (e >= nel)
                     continue;
-                // stages 1 and 4: the LDS value already holds the own part and c1 times the
-                // commutator and same terms; f gathers the neighbour terms alone
-                const C lv = sig[lo[u]];
-                C f = (STAGE == 1 || STAGE == 4) ? mk2<R>(R(0), R(0)) : lv;
-#pragma unroll
-                for (int k = 0; k < NT; ++k) {
-                    const TermT<R> t = terms[e2[u] * NT + k];
-                    const int v = nbv[u][k].x & 63;
-                    if constexpr (PLUS) {
-                        const R cp = t.plus_c * sqrt_n[v + 1];
-                        f.x = fma(-cp, xp[u][k].y, f.x);
-                        f.y = fma(cp, xp[u][k].x, f.y);
-                    }
-                    const R sm = sqrt_n[v];
-                    f = cfma(t.minus_c, mk2<R>(sm * xm[u][k].x, sm * xm[u][k].y), f);
-                }
+                const C f = sig[place(k)];
                 C r0, r1 = mk2<R>(R(0), R(0));
                 if (STAGE == 1) {
-                    r0 = mk2<R>(fma(a.c1, f.x, lv.x), fma(a.c1, f.y, lv.y));
+                    r0 = f;
                 } else if (STAGE == 4) {
                     constexpr R third = R(1) / R(3);
-                    r0 = mk2<R>(fma(ep[u].x, third, fma(a.c1, f.x, lv.x)), fma(ep[u].y, third, fma(a.c1, f.y, lv.y)));
+                    r0 = mk2<R>(fma(ep[k].x, third, f.x), fma(ep[k].y, third, f.y));
                 } else {
-                    stage_values<STAGE, R>(a.c1, STAGE == 2 ? own[u] : mk2<R>(R(0), R(0)), f, ep[u], r0, r1);
+                    stage_values<STAGE, R>(a.c1, STAGE == 2 ? own[k] : mk2<R>(R(0), R(0)), f,
+                                           STAGE == 2 || STAGE == 3 ? ep[k] : mk2<R>(R(0), R(0)), r0, r1);
                 }
-                stage_store<STAGE, R>(a, o[u], r0, r1);
+                if (live)
+                    stage_store<STAGE, R>(a, q * nel + e, r0, r1);
+            }
+            wave_sync();
+            if (!ONE && !EARLY)
+                ahead(false, true);
+        }
+        if (ONE || q0n < 0)
+            break;
+        q0 = q0n;
+    }
+}
+
+// One iteration of the thermal state search (tss.hip): y_u = C^T [ (C k_u C^T) / D_u ] C with
+// k = f_TSS(y), the "same" and neighbour terms alone; the matrix stays in LDS through the four
+// products.
+template <int SZ, bool REALC, bool WLDS>
+__global__ __launch_bounds__(kWideThreads) void tss_iteration_wide(StageArgsT<double> a, WideTables<double> wt,
+                                                                   WideTss ts, const double2* __restrict__ gam_all,
+                                                                   int N, int T)
+{
+    using C = double2;
+    using TM = std::conditional_t<REALC, double, C>;
+    constexpr int NB = (SZ + 15) / 16, NL = (SZ * SZ + 63) / 64, NP = wide_pitch(SZ);
+    extern __shared__ __align__(16) unsigned char wide_mem[];
+    const int nel = N * N;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int terms = wt.W * wt.len;
+    constexpr bool GL = kWideGamLds<double, SZ>;
+    const WideLds L = wide_lds(N, (int)sizeof(C), REALC, GL, T, WLDS ? terms * 4 : 0);
+    TM* cl = reinterpret_cast<TM*>(wide_mem);
+    C* gl = reinterpret_cast<C*>(wide_mem + L.gam);
+    uint32_t* el = reinterpret_cast<uint32_t*>(wide_mem + L.where);
+    C* sig = reinterpret_cast<C*>(wide_mem + L.mat) + (int64_t)w * (N * NP);
+    int places[(NL + 1) / 2];  // of this lane's elements, two to a register
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
+        const int at = wt.place[min(lane + 64 * k, nel - 1)];
+        places[k / 2] = k & 1 ? places[k / 2] | at << 16 : at;
+    }
+    auto place = [&](int k) { return k & 1 ? (int)((uint32_t)places[k / 2] >> 16) : places[k / 2] & 0xffff; };
+    const double sq_lane = sqrt((double)lane);
+
+    const Walk walk(wt.tile_order, a.ntiles, T);
+    int inst = -1, cls = -1;
+    for (int j = walk.j;; j += walk.gx) {
+        const int64_t q0 = walk.group<false>(j), q = q0 + w;
+        if (q0 < 0)
+            break;
+        const int it = a.tile_inst ? a.tile_inst[q0 / kTile] : 0;
+        const int cc = tile_bath_class(a, (int)(q0 / kTile));
+        const C* gam = gam_all + (int64_t)cc * nel;
+        const uint32_t* where = wt.where + (int64_t)cc * terms;
+        if (it != inst || cc != cls)
+            load_constants<double, TM, SZ, WLDS>(ts.c + (int64_t)it * nel, gam, where, terms, N, cl, gl, el, inst < 0);
+        inst = it;
+        cls = cc;
+        if (q >= a.zero_slot)
+            continue;
+        EdgeLanes ed;
+        ed.load(a.nb, a.mp, q, lane, wt.W, a.zero_slot);
+        const C S = a.pfss[q], em = ts.epsm[q];
+#pragma unroll
+        for (int k = 0; k < NL; ++k) {
+            const int e = lane + 64 * k;
+            if (e < nel) {
+                const int at = place(k);
+                const C g = GL ? gl[at] : gam[at / NP * N + at % NP], y = a.yin[q * nel + e];
+                sig[at] = cfma(mk2<double>(S.x + g.x, S.y + g.y), y, mk2<double>(0.0, 0.0));
             }
         }
+        wave_sync();
+        Neighbours<double, kWideModesAhead<double, SZ, true>> nbs(a, wt, cc, WLDS ? el : where, ed, q, nel, lane);
+        nbs.template run<false>(1.0, sq_lane, sig);
+        wave_sync();
+        const C* w_ij = ts.w + (int64_t)it * nel;
+        auto put = [&](int at, int, int, C v) {
+            sig[at] = v;
+            return v;
+        };
+        Product<double, NB> p;
+        p.clear();
+        multiply<true, false, false, double, NB, NP>(p, sig, cl, N, lane);  // C k
+        wave_sync();
+        each_element<double, NB, NP>(p, N, lane, put);
+        wave_sync();
+        p.clear();
+        multiply<false, true, false, double, NB, NP>(p, sig, cl, N, lane);  // (C k) C^T
+        wave_sync();
+        each_element<double, NB, NP>(p, N, lane, [&](int at, int i, int jj, C v) {
+            const C wij = w_ij[i * N + jj];
+            const C d = mk2<double>(wij.x + em.x, wij.y + em.y);
+            const double den = d.x * d.x + d.y * d.y;
+            return put(at, i, jj, mk2<double>((v.x * d.x + v.y * d.y) / den, (v.y * d.x - v.x * d.y) / den));
+        });
+        wave_sync();
+        p.clear();
+        multiply<true, true, false, double, NB, NP>(p, sig, cl, N, lane);  // C^T B
+        wave_sync();
+        each_element<double, NB, NP>(p, N, lane, put);
+        wave_sync();
+        p.clear();
+        multiply<false, false, false, double, NB, NP>(p, sig, cl, N, lane);  // (C^T B) C
+        wave_sync();
+        each_element<double, NB, NP>(p, N, lane, put);
+        wave_sync();
+        const bool pad = ts.q2u[q] < 0;
+#pragma unroll
+        for (int k = 0; k < NL; ++k) {
+            const int e = lane + 64 * k;
+            if (e < nel)
+                nt_store<double>(pad ? mk2<double>(0.0, 0.0) : sig[place(k)], a.yout + q * nel + e);
+        }
+        wave_sync();
+    }
+}
+
+// How a launch is divided: T wavefronts per workgroup (`ados` where a caller chose), and a
+// workgroup per group of T ADOs where all of them fit the card at once (`one`; the tiles are
+// dealt to the XCDs whole, so the XCD with the most tiles sets the number), or as many as run
+// at once.
+struct WideShape {
+    int T;
+    bool one;
+    unsigned wgs;
+};
+template <typename R, int SZ>
+WideShape wide_shape(int N, bool real, int W, int len, int ntiles, int ados)
+{
+    const auto shape = [&](int T) {
+        const int64_t all = (int64_t)(ntiles + kNumXcd - 1) / kNumXcd * kNumXcd * (kTile / T);
+        const int64_t most = (int64_t)kWideCus * 4 * kWideOccupancy<R, SZ> / T;
+        return WideShape{T, all <= most, (unsigned)std::min(all, most)};
     };
-    if (tile_has_plus(a, (int)(q0 / kTile)))
-        phase_c(std::true_type{});
-    else
-        phase_c(std::false_type{});
+    const auto lds = [&](int T) {
+        return wide_lds(N, (int)sizeof(c2<R>), real, kWideGamLds<R, SZ>, T, wide_where_bytes(W, len)).total;
+    };
+    const int fit = wide_tile(N, (int)sizeof(c2<R>), W);
+    if (ados > 0 && ados <= fit && kTile % ados == 0)
+        return shape(ados);
+    // 4, as many as a CU's SIMDs; 8 where the CU's LDS does not hold two such workgroups and
+    // each wavefront has several ADOs to go through (32 sites, ms per RK4 step in complex128:
+    // 6,545 ADOs 0.640 with 4, 0.582 with 8; 561 ADOs 0.101 and 0.133)
+    const WideShape four = shape(std::min(fit, 4));
+    return !four.one && 2 * lds(4) > kWideLdsAll && lds(8) <= kWideLdsAll ? shape(8) : four;
 }
 
-template <typename R, int B, int NT, bool REALH, int LDSB>
-void launch_wl(int N, int stage, const StageArgsT<R>& a, const ElementArgsT<R>& el, int T, hipStream_t st)
+template <typename R, int SZ, bool REALH, bool ONE, bool WLDS>
+void launch_wo(int N, int stage, const StageArgsT<R>& a, const ElementArgsT<R>& el, const WideTables<R>& wt,
+               WideShape sh, hipStream_t st)
 {
-    const dim3 grid((unsigned)(a.mp / T)), block(64 * T);
+    const int T = sh.T;
+    const dim3 grid(sh.wgs), block(64 * T);
+    const size_t lds =
+        (size_t)wide_lds(N, (int)sizeof(c2<R>), REALH, kWideGamLds<R, SZ>, T, wide_where_bytes(wt.W, wt.len)).total;
     switch (stage) {
-    case 0: hipLaunchKernelGGL((rk4_stage_wide<R, B, NT, 0, REALH, LDSB>), grid, block, 0, st, a, el.hs, el.gam, el.terms, N, T); break;
-    case 1: hipLaunchKernelGGL((rk4_stage_wide<R, B, NT, 1, REALH, LDSB>), grid, block, 0, st, a, el.hs, el.gam, el.terms, N, T); break;
-    case 2: hipLaunchKernelGGL((rk4_stage_wide<R, B, NT, 2, REALH, LDSB>), grid, block, 0, st, a, el.hs, el.gam, el.terms, N, T); break;
-    case 3: hipLaunchKernelGGL((rk4_stage_wide<R, B, NT, 3, REALH, LDSB>), grid, block, 0, st, a, el.hs, el.gam, el.terms, N, T); break;
-    default: hipLaunchKernelGGL((rk4_stage_wide<R, B, NT, 4, REALH, LDSB>), grid, block, 0, st, a, el.hs, el.gam, el.terms, N, T); break;
+    case 0: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 0, REALH, ONE, WLDS>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
+    case 1: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 1, REALH, ONE, WLDS>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
+    case 2: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 2, REALH, ONE, WLDS>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
+    case 3: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 3, REALH, ONE, WLDS>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
+    default: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 4, REALH, ONE, WLDS>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
     }
 }
 
-// the LDS instance: H and T matrices of N x wide_row(N) complex elements
-template <typename R, int B, int NT, bool REALH>
-void launch_wb(int N, int stage, const StageArgsT<R>& a, const ElementArgsT<R>& el, int T, hipStream_t st)
+template <typename R, int SZ, bool REALH>
+void launch_ws(int N, int stage, const StageArgsT<R>& a, const ElementArgsT<R>& el, const WideTables<R>& wt, int ados,
+               hipStream_t st)
 {
-    if (wide_lds_bytes(N, (int)sizeof(c2<R>), 2 * a.table_units - 2, T) <= kWideLdsSmallBytes)
-        launch_wl<R, B, NT, REALH, kWideLdsSmallBytes>(N, stage, a, el, T, st);
+    const WideShape sh = wide_shape<R, SZ>(N, REALH, wt.W, wt.len, a.ntiles, ados);
+    if (wide_where_bytes(wt.W, wt.len) == 0)
+        launch_wo<R, SZ, REALH, false, false>(N, stage, a, el, wt, sh, st);
+    else if (sh.one)
+        launch_wo<R, SZ, REALH, true, true>(N, stage, a, el, wt, sh, st);
     else
-        launch_wl<R, B, NT, REALH, kWideLdsBytes>(N, stage, a, el, T, st);
-}
-
-template <typename R, int B, bool REALH>
-void launch_wn(int N, int nt, int stage, const StageArgsT<R>& a, const ElementArgsT<R>& el, int T, hipStream_t st)
-{
-    switch (nt) {
-    case 2: launch_wb<R, B, 2, REALH>(N, stage, a, el, T, st); break;
-    case 4: launch_wb<R, B, 4, REALH>(N, stage, a, el, T, st); break;
-    default: launch_wb<R, B, 8, REALH>(N, stage, a, el, T, st); break;
-    }
+        launch_wo<R, SZ, REALH, false, true>(N, stage, a, el, wt, sh, st);
 }
 
 template <typename R, bool REALH>
-void launch_w(int N, int nt, int stage, const StageArgsT<R>& a, const ElementArgsT<R>& el, int ados, hipStream_t st)
+void launch_w(int N, int stage, const StageArgsT<R>& a, const ElementArgsT<R>& el, const WideTables<R>& wt, int ados,
+              hipStream_t st)
 {
-    const int fit = wide_tile(N, (int)sizeof(c2<R>), 2 * a.table_units - 2);
-    const int T = ados > 0 && ados <= fit && kTile % ados == 0 ? ados : fit;
-    const int B = (N + 7) / 8;
-    if (B <= 2)
-        launch_wn<R, 2, REALH>(N, nt, stage, a, el, T, st);
-    else if (B == 3)
-        launch_wn<R, 3, REALH>(N, nt, stage, a, el, T, st);
+    if (N <= 16)
+        launch_ws<R, 16, REALH>(N, stage, a, el, wt, ados, st);
+    else if (N <= 24)
+        launch_ws<R, 24, REALH>(N, stage, a, el, wt, ados, st);
     else
-        launch_wn<R, 4, REALH>(N, nt, stage, a, el, T, st);
+        launch_ws<R, 32, REALH>(N, stage, a, el, wt, ados, st);
+}
+
+template <int SZ, bool REALC>
+void launch_tr(int N, const StageArgsT<double>& a, const double2* gam, const WideTables<double>& wt, const WideTss& ts,
+               hipStream_t st)
+{
+    const WideShape sh = wide_shape<double, SZ>(N, REALC, wt.W, wt.len, a.ntiles, 0);
+    const int wb = wide_where_bytes(wt.W, wt.len), T = sh.T;
+    const size_t lds = (size_t)wide_lds(N, (int)sizeof(double2), REALC, kWideGamLds<double, SZ>, T, wb).total;
+    const dim3 grid(sh.wgs), block(64 * T);
+    if (wb)
+        hipLaunchKernelGGL((tss_iteration_wide<SZ, REALC, true>), grid, block, lds, st, a, wt, ts, gam, N, T);
+    else
+        hipLaunchKernelGGL((tss_iteration_wide<SZ, REALC, false>), grid, block, lds, st, a, wt, ts, gam, N, T);
+}
+
+template <int SZ>
+void launch_ts(int N, bool real_c, const StageArgsT<double>& a, const double2* gam, const WideTables<double>& wt,
+               const WideTss& ts, hipStream_t st)
+{
+    if (real_c)
+        launch_tr<SZ, true>(N, a, gam, wt, ts, st);
+    else
+        launch_tr<SZ, false>(N, a, gam, wt, ts, st);
 }
 
 }  // namespace
@@ -314,22 +902,33 @@ bool wide_supported(int N, int complex_bytes, int W)
 
 int wide_max_ados(int N, int complex_bytes, int W) { return wide_tile(N, complex_bytes, W); }
 
-void launch_stage_wide(int N, int nterm_slots, bool real_h, int stage, const StageArgsT<double>& a,
-                       const ElementArgsT<double>& el, int ados, hipStream_t s)
+void launch_stage_wide(int N, bool real_h, int stage, const StageArgsT<double>& a, const ElementArgsT<double>& el,
+                       const WideTables<double>& wt, int ados, hipStream_t s)
 {
     if (real_h)
-        launch_w<double, true>(N, nterm_slots, stage, a, el, ados, s);
+        launch_w<double, true>(N, stage, a, el, wt, ados, s);
     else
-        launch_w<double, false>(N, nterm_slots, stage, a, el, ados, s);
+        launch_w<double, false>(N, stage, a, el, wt, ados, s);
 }
 
-void launch_stage_wide(int N, int nterm_slots, bool real_h, int stage, const StageArgsT<float>& a,
-                       const ElementArgsT<float>& el, int ados, hipStream_t s)
+void launch_stage_wide(int N, bool real_h, int stage, const StageArgsT<float>& a, const ElementArgsT<float>& el,
+                       const WideTables<float>& wt, int ados, hipStream_t s)
 {
     if (real_h)
-        launch_w<float, true>(N, nterm_slots, stage, a, el, ados, s);
+        launch_w<float, true>(N, stage, a, el, wt, ados, s);
     else
-        launch_w<float, false>(N, nterm_slots, stage, a, el, ados, s);
+        launch_w<float, false>(N, stage, a, el, wt, ados, s);
+}
+
+void launch_tss_wide(int N, bool real_c, const StageArgsT<double>& a, const double2* gam, const WideTables<double>& wt,
+                     const WideTss& ts, hipStream_t s)
+{
+    if (N <= 16)
+        launch_ts<16>(N, real_c, a, gam, wt, ts, s);
+    else if (N <= 24)
+        launch_ts<24>(N, real_c, a, gam, wt, ts, s);
+    else
+        launch_ts<32>(N, real_c, a, gam, wt, ts, s);
 }
 
 }  // namespace heom_hip

@@ -13,10 +13,11 @@
 //
 // k needs no kernel of its own: eps y is the S_u y term of the ordinary RHS with S_u = eps
 // for every ADO and H = 0, so a search handle is an ordinary handle built from such a
-// descriptor, whose stage kernels (STAGE 0, one evaluation, y -> ya) compute f_TSS
-// unchanged.  The transform runs per ADO in one kernel for N <= 8 (a tile of 64 ADOs in
-// LDS, one wavefront per matrix row; C, C^T and (i/hbar)(E_i - E_j) are wave-uniform)
-// and in four passes over out-of-place planes for 8 < N <= 32.
+// descriptor, whose stage kernels (STAGE 0, one evaluation) compute f_TSS unchanged for
+// heom_rhs.  An iteration is one kernel that leaves out the commutator of H = 0 and keeps k
+// and the four products on the CU: here for N <= 8 (a tile of 64 ADOs in LDS), in
+// stage_wide.hip for 8 < N <= 32 (a matrix per wavefront).  It reads the state and writes the
+// next one into the work buffer; the two then exchange their places.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -232,42 +233,6 @@ __global__ __launch_bounds__(64 * N) void tss_iteration(TssArgs a, const double2
         tss_tile<N, NT, TC, false>(a, gam, terms, modes, c + off, ct + off, wd + off, tile, t);
 }
 
-// 8 < N <= 32, one pass, thread = (element e, slot q):
-//   left:  out[e][q] = sum_m mx[i][m] in[m*N+j][q]
-//   right: out[e][q] = sum_m in[i*N+m][q] mx[m][j]   (divided by D when w is given)
-__global__ void tss_pass(const double2* __restrict__ in, double2* __restrict__ out, const double2* __restrict__ mx,
-                         const double2* __restrict__ w, const double2* __restrict__ epsm,
-                         const int32_t* __restrict__ q2u, const int32_t* __restrict__ tile_inst, int64_t mp, int N,
-                         int left)
-{
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int nel = N * N;
-    if (t >= (int64_t)nel * mp)
-        return;
-    const int e = (int)(t / mp);
-    const int64_t q = t % mp;
-    const int i = e / N, j = e % N;
-    if (tile_inst) {
-        const int64_t off = (int64_t)tile_inst[q / kTile] * nel;
-        mx += off;
-        if (w)
-            w += off;
-    }
-    double2 v = make_double2(0.0, 0.0);
-    if (left) {
-        for (int m = 0; m < N; ++m)
-            v = cfma(mx[i * N + m], in[(int64_t)(m * N + j) * mp + q], v);
-    } else {
-        for (int m = 0; m < N; ++m)
-            v = cfma(in[(int64_t)(i * N + m) * mp + q], mx[m * N + j], v);
-    }
-    if (w) {
-        const double2 em = epsm[q];
-        v = cdiv(v, make_double2(w[e].x + em.x, w[e].y + em.y));
-    }
-    out[t] = q2u[q] < 0 ? make_double2(0.0, 0.0) : v;
-}
-
 template <int N, int NT>
 void launch_iteration_t(heom_handle* h, const TssArgs& a)
 {
@@ -468,8 +433,6 @@ int heom_tss_step(heom_handle* h, int64_t n)
         const TssState& T = *h->tss;
         const int N = h->N;
         const int32_t* ti = h->count > 1 ? h->tile_inst.p : nullptr;
-        const int64_t total = (int64_t)h->nel * h->Mp;
-        const dim3 pgrid(blocks_for(total, 256)), pblock(256);
         for (int64_t s = 0; s < n; ++s) {
             if (N <= kMaxStates) {
                 // y -> ya, then the two exchange their places
@@ -491,16 +454,12 @@ int heom_tss_step(heom_handle* h, int64_t n)
                 h->timing.rhs_launches += 1;
                 continue;
             }
-            double2* y = h->y.as<double2>();
-            double2* ya = h->ya.as<double2>();
-            double2* yb = h->yb.as<double2>();
-            launch_stage_buffers(h, 0, h->y.p, h->y.p, h->pbuf.p, h->ya.p, 0.0, false, false);
-            // C k -> yb, (. C^T) / D -> ya, C^T . -> yb, . C -> y, in the reference's order
-            hipLaunchKernelGGL(tss_pass, pgrid, pblock, 0, h->stream, ya, yb, T.c.p, nullptr, nullptr, h->q2u.p, ti, h->Mp, N, 1);
-            hipLaunchKernelGGL(tss_pass, pgrid, pblock, 0, h->stream, yb, ya, T.ct.p, T.w.p, T.epsm.p, h->q2u.p, ti, h->Mp, N, 0);
-            hipLaunchKernelGGL(tss_pass, pgrid, pblock, 0, h->stream, ya, yb, T.ct.p, nullptr, nullptr, h->q2u.p, ti, h->Mp, N, 1);
-            hipLaunchKernelGGL(tss_pass, pgrid, pblock, 0, h->stream, yb, y, T.c.p, nullptr, nullptr, h->q2u.p, ti, h->Mp, N, 0);
+            const StageArgsT<double> a = stage_args64(h, h->y.p, h->y.p, h->pbuf.p, h->ya.p, 0.0, false);
+            launch_tss_wide(N, T.real_c, a, h->gam.p, h->wide_tables<double>(),
+                            WideTss{T.c.p, T.w.p, T.epsm.p, h->q2u.p}, h->stream);
             HIPC(hipGetLastError());
+            std::swap(h->y.p, h->ya.p);
+            h->timing.rhs_launches += 1;
         }
     });
 }
