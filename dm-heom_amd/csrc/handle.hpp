@@ -193,8 +193,8 @@ struct heom_handle {
     // N > 8: the neighbour terms by mode (WideTables), [classes][W][wide_len]
     DevBuf<Term> wterms;
     DevBuf<TermT<float>> wterms32;
-    DevBuf<uint32_t> wwhere;
-    DevBuf<uint16_t> wplace;  // [N*N]
+    DevBuf<uint32_t> wwhere;     // then, from entry wide_place on, the places of the positions
+    size_t wide_place = 0;
     DevBuf<int32_t> tile_order;  // tiles with plus neighbours first
     int wide_len = 0;
     int S = 0;                    // tier-0/1 ADOs
@@ -230,10 +230,11 @@ struct heom_handle {
     template <typename R>
     heom_hip::WideTables<R> wide_tables() const
     {
+        const uint16_t* places = reinterpret_cast<const uint16_t*>(wwhere.p + wide_place);
         if constexpr (sizeof(R) == sizeof(double))
-            return {wterms.p, wwhere.p, tile_order.p, wplace.p, W, wide_len};
+            return {wterms.p, wwhere.p, tile_order.p, places, W, wide_len};
         else
-            return {wterms32.p, wwhere.p, tile_order.p, wplace.p, W, wide_len};
+            return {wterms32.p, wwhere.p, tile_order.p, places, W, wide_len};
     }
     size_t cbytes() const { return fp32() ? sizeof(float2) : sizeof(double2); }
 

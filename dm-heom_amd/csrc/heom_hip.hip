@@ -798,7 +798,6 @@ void build_tile_plus(heom_handle* h, const std::vector<int2>& nb)
                 if (f[(size_t)t] == want)
                     order.push_back(t);
         upload(h->tile_order, order, h->stream);
-        HIPC(hipStreamSynchronize(h->stream));
     }
 }
 
@@ -933,11 +932,13 @@ void build_wide_terms(heom_handle* h, const std::vector<std::vector<Term>>& per,
             where[m * len + k] = (uint32_t)wide_pos(N, i, j) | (uint32_t)(i * wide_pitch(N) + j) << 16;
         }
     }
-    std::vector<uint16_t> place((size_t)nel);
+    // one allocation and copy for both: the places follow the modes' entries
+    h->wide_place = where.size();
+    where.resize(where.size() + ((size_t)nel + 1) / 2);
+    uint16_t* place = reinterpret_cast<uint16_t*>(where.data() + h->wide_place);
     for (int i = 0; i < N; ++i)
         for (int j = 0; j < N; ++j)
             place[(size_t)wide_pos(N, i, j)] = (uint16_t)(i * wide_pitch(N) + j);
-    upload(h->wplace, place, h->stream);
     upload(h->wwhere, where, h->stream);
     if (h->fp32()) {
         std::vector<TermT<float>> f32(flat.size());
@@ -945,10 +946,8 @@ void build_wide_terms(heom_handle* h, const std::vector<std::vector<Term>>& per,
             f32[t] = {make_float2((float)flat[t].minus_c.x, (float)flat[t].minus_c.y), (float)flat[t].plus_c,
                       flat[t].mode, flat[t].info};
         upload(h->wterms32, f32, h->stream);
-        HIPC(hipStreamSynchronize(h->stream));
     } else {
         upload(h->wterms, flat, h->stream);
-        HIPC(hipStreamSynchronize(h->stream));
     }
 }
 
@@ -2247,7 +2246,7 @@ int heom_device_bytes(heom_handle* h, int64_t* bytes)
         if (!bytes)
             raise(HEOM_E_INVALID, "bytes is NULL");
         int64_t b = h->y.bytes() + h->pbuf.bytes() + h->ya.bytes() + h->yb.bytes();
-        b += h->wterms.bytes() + h->wterms32.bytes() + h->wwhere.bytes();
+        b += h->wterms.bytes() + h->wterms32.bytes() + h->wwhere.bytes() + h->tile_order.bytes();
         for (auto* x : {&h->pfss, &h->hs, &h->gam, &h->mx, &h->small, &h->y64, &h->sa64, &h->sb64, &h->p64,
                         &h->sp_pfss, &h->sp_tmp})
             b += x->bytes();
