@@ -17,6 +17,11 @@
 // The wavefronts of a workgroup share only H / hbar and the "same" constants in LDS, so there
 // is a barrier only where the instance changes; the LDS accesses of one wavefront complete
 // in order.
+// Measured at 24 sites, 20,475 ADOs (ms per RK4 step; before: workgroups of 4 ADOs on element
+// planes, every element's term list with a missing neighbour's zeros read as well): 1.008 ->
+// 0.668 in complex128, 0.697 -> 0.449 in complex64; at 9 sites, 715 ADOs, 0.0280 -> 0.0266.  A
+// wavefront's own instructions bound it (some 400 cycles an edge), not memory: the state's 12
+// passes take 0.451 and 0.225 ms at the rate of a large copy.
 #include <algorithm>
 #include <type_traits>
 
@@ -536,9 +541,8 @@ __device__ __forceinline__ void load_constants(const c2<R>* __restrict__ m, cons
 // One RK4 stage (STAGE 1..4, or 0: the RHS alone) over the whole hierarchy.  N <= SZ.
 template <typename R, int SZ, int STAGE, bool REALH, bool ONE, bool WLDS>
 __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(kWideOccupancy<R, SZ>)))
-void rk4_stage_wide(StageArgsT<R> a, WideTables<R> wt,
-                                                               const c2<R>* __restrict__ hs_all,
-                                                               const c2<R>* __restrict__ gam_all, int N_, int T)
+void rk4_stage_wide(StageArgsT<R> a, WideTables<R> wt, const c2<R>* __restrict__ hs_all,
+                    const c2<R>* __restrict__ gam_all, int N_, int T)
 {
     using C = c2<R>;
     using TM = std::conditional_t<REALH, R, C>;
@@ -552,7 +556,9 @@ void rk4_stage_wide(StageArgsT<R> a, WideTables<R> wt,
     // needs its own values to the end and loads the next ones after that)
     constexpr bool EARLY = STAGE != 2 && NL * sizeof(C) <= 144;
     extern __shared__ __align__(16) unsigned char wide_mem[];
-    // one round trip for the arguments that the first loads need, not one at each of them
+    // one round trip for the arguments that the first loads need, not one at each of them (9
+    // sites, 715 ADOs: 0.0285 -> 0.0268 ms per RK4 step); not in the longer kernels, which
+    // have no scalar registers to spare
     if (ONE)
         asm volatile("" ::"s"(a.yin), "s"(a.nb), "s"(a.mp), "s"(a.pfss), "s"(a.tile_inst), "s"(a.tile_class), "s"(wt.place),
                      "s"(wt.where), "s"(wt.terms), "s"(wt.W), "s"(wt.len), "s"(hs_all), "s"(gam_all), "s"(N_), "s"(T),
@@ -694,7 +700,7 @@ void rk4_stage_wide(StageArgsT<R> a, WideTables<R> wt,
 
 // One iteration of the thermal state search (tss.hip): y_u = C^T [ (C k_u C^T) / D_u ] C with
 // k = f_TSS(y), the "same" and neighbour terms alone; the matrix stays in LDS through the four
-// products.
+// products (24 sites, 2,925 ADOs: 241 us an iteration as a stage launch and four passes, 57 us so).
 template <int SZ, bool REALC, bool WLDS>
 __global__ __launch_bounds__(kWideThreads) void tss_iteration_wide(StageArgsT<double> a, WideTables<double> wt,
                                                                    WideTss ts, const double2* __restrict__ gam_all,

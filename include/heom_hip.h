@@ -322,7 +322,7 @@ typedef struct heom_tune_result {
     int32_t kernel;              /* enum heom_stage_kind */
     int32_t xcd_chunk;           /* tiles per XCD chunk of the tile order */
     int32_t workgroups;          /* pipelined kernel: persistent workgroups, else 0 */
-    int32_t ados_per_workgroup;  /* 64, or the wide kernel's ADOs per workgroup */
+    int32_t ados_per_workgroup;  /* 64, or the wide kernel's ADOs (wavefronts) per workgroup */
     int32_t chosen;              /* 1 for the configuration kept */
     int32_t tile_split;          /* tile kernel: workgroups per 64-ADO tile (1, 2 or 4), else 1 */
     double ms_per_step;          /* device time of one RK4 step */
