@@ -700,7 +700,7 @@ void rk4_stage_wide(StageArgsT<R> a, WideTables<R> wt, const c2<R>* __restrict__
 
 // One iteration of the thermal state search (tss.hip): y_u = C^T [ (C k_u C^T) / D_u ] C with
 // k = f_TSS(y), the "same" and neighbour terms alone; the matrix stays in LDS through the four
-// products (24 sites, 2,925 ADOs: 241 us an iteration as a stage launch and four passes, 57 us so).
+// products (24 sites, 2,925 ADOs: 241 us an iteration as a stage launch and four passes, 54 us so).
 template <int SZ, bool REALC, bool WLDS>
 __global__ __launch_bounds__(kWideThreads) void tss_iteration_wide(StageArgsT<double> a, WideTables<double> wt,
                                                                    WideTss ts, const double2* __restrict__ gam_all,
@@ -772,15 +772,33 @@ __global__ __launch_bounds__(kWideThreads) void tss_iteration_wide(StageArgsT<do
         wave_sync();
         each_element<double, NB, NP>(p, N, lane, put);
         wave_sync();
+        // the denominators' part of this lane's elements, all of them under way during the
+        // product (one at a time they were a round trip each: 24 sites, 2,925 ADOs 57 -> 54 us
+        // an iteration); 32 x 32 matrices spill with them (32 sites, depth 3: 157 us, 161 so)
+        constexpr bool kDenAhead = SZ <= 24;
+        vec2_t<double> wv[kDenAhead ? NB * NB * 4 : 1];
+        if constexpr (kDenAhead) {
+#pragma unroll
+            for (int t = 0; t < NB * NB * 4; ++t) {
+                const int i = min(16 * (t / (4 * NB)) + d_row<double>(lane, t % 4), N - 1);
+                const int jj = min(16 * (t / 4 % NB) + (lane & 15), N - 1);
+                wv[t] = *reinterpret_cast<const vec2_t<double>*>(w_ij + i * N + jj);
+            }
+        }
         p.clear();
         multiply<false, true, false, double, NB, NP>(p, sig, cl, N, lane);  // (C k) C^T
         wave_sync();
-        each_element<double, NB, NP>(p, N, lane, [&](int at, int i, int jj, C v) {
-            const C wij = w_ij[i * N + jj];
-            const C d = mk2<double>(wij.x + em.x, wij.y + em.y);
-            const double den = d.x * d.x + d.y * d.y;
-            return put(at, i, jj, mk2<double>((v.x * d.x + v.y * d.y) / den, (v.y * d.x - v.x * d.y) / den));
-        });
+#pragma unroll
+        for (int t = 0; t < NB * NB * 4; ++t) {
+            const int ta = t / (4 * NB), tb = t / 4 % NB, i = 16 * ta + d_row<double>(lane, t % 4), jj = 16 * tb + (lane & 15);
+            const C v = mk2<double>(p.re[ta][tb][t % 4], p.im[ta][tb][t % 4]);
+            if (i < N && jj < N) {
+                const C wij = kDenAhead ? mk2<double>(wv[kDenAhead ? t : 0].x, wv[kDenAhead ? t : 0].y) : w_ij[i * N + jj];
+                const C d = mk2<double>(wij.x + em.x, wij.y + em.y);
+                const double den = d.x * d.x + d.y * d.y;
+                sig[i * NP + jj] = mk2<double>((v.x * d.x + v.y * d.y) / den, (v.y * d.x - v.x * d.y) / den);
+            }
+        }
         wave_sync();
         p.clear();
         multiply<true, true, false, double, NB, NP>(p, sig, cl, N, lane);  // C^T B
