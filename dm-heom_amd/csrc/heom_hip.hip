@@ -801,6 +801,17 @@ void build_tile_plus(heom_handle* h, const std::vector<int2>& nb)
     }
 }
 
+// the bath class of each tile, by its instance (only where the classes differ)
+void upload_tile_class(heom_handle* h, const std::vector<int32_t>& tinst)
+{
+    if (h->uniform)
+        return;
+    std::vector<int32_t> tcls(tinst.size());
+    for (size_t t = 0; t < tinst.size(); ++t)
+        tcls[t] = h->inst_class[(size_t)tinst[t]];
+    upload(h->tile_class, tcls, h->stream);
+}
+
 // H [count][N*N*2] in J -> H / hbar on the device
 void set_hamiltonians(heom_handle* h, const double* H)
 {
@@ -1383,13 +1394,9 @@ void create_batch(heom_handle* h, const heom_desc* d, int count)
     upload(h->q2u, q2u, h->stream);
     upload(h->tile_inst, tinst, h->stream);
     upload(h->q_top, qtop, h->stream);
-    if (!h->uniform) {
-        std::vector<int32_t> tcls(h->ntiles, h->inst_class[count - 1]);
-        for (int t = 0; t < h->ntiles; ++t)
-            tcls[t] = h->inst_class[tinst[t]];
-        upload(h->tile_class, tcls, h->stream);
+    upload_tile_class(h, tinst);
+    if (!h->uniform)
         upload(h->inst_class_d, h->inst_class, h->stream);
-    }
     if (h->fp32()) {
         std::vector<float2> p32(Mp);
         for (int64_t q = 0; q < Mp; ++q)
@@ -2378,6 +2385,7 @@ int heom_compact(heom_handle* h, int64_t* active)
         upload(h->nb, nb_n, h->stream);
         upload(h->q2u, q2u_n, h->stream);
         upload(h->tile_inst, tinst, h->stream);
+        upload_tile_class(h, tinst);
         upload(h->q_top, qtop, h->stream);
         h->Mp = mp;
         h->ntiles = ntiles;
