@@ -382,6 +382,10 @@ struct WideTss {
     const double2* __restrict__ epsm;
     const int32_t* __restrict__ q2u;
 };
+// workgroups of a kernel that goes through mp slots, each by one of kMatrixThreads: a launch
+// has fewer than 2^32 threads, which one workgroup per slot passes at 16.8 million slots
+constexpr int kMatrixThreads = 256;
+constexpr unsigned matrix_blocks(int64_t mp) { return (unsigned)(mp < (1 << 20) ? mp : 1 << 20); }
 // W: bath modes
 bool wide_supported(int N, int complex_bytes, int W);
 // the largest number of wavefronts (ADOs at a time) per workgroup, a power of two <= 8

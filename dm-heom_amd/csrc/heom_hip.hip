@@ -69,22 +69,23 @@ __device__ __forceinline__ int64_t plane_index(bool paired, int N, int e, int64_
     return c64_index(sizeof(C) == sizeof(float2) && paired, N, e, q, mp);
 }
 
-// Matrix-major states (N > kMaxStates): a copy of whole matrices between the two orders,
-// one workgroup per slot q; TO_STATE: dst[q] = src[u(q)] (0 for a slot without an ADO),
+// Matrix-major states (N > kMaxStates): a copy of whole matrices between the two orders, a
+// workgroup per slot q at a time; TO_STATE: dst[q] = src[u(q)] (0 for a slot without an ADO),
 // otherwise dst[u(q)] = src[q]
 template <typename C, bool TO_STATE>
 __global__ void copy_matrices(const double2* __restrict__ uid_order, C* __restrict__ state,
-                              double2* __restrict__ uid_out, const int32_t* __restrict__ q2u, int N)
+                              double2* __restrict__ uid_out, const int32_t* __restrict__ q2u, int64_t mp, int N)
 {
-    const int64_t q = blockIdx.x;
-    const int32_t u = q2u[q];
     const int nel = N * N;
-    for (int e = threadIdx.x; e < nel; e += blockDim.x) {
-        const int64_t at = q * nel + wide_pos(N, e / N, e % N);
-        if (TO_STATE)
-            state[at] = from_d2<C>(u >= 0 ? uid_order[(int64_t)u * nel + e] : make_double2(0.0, 0.0));
-        else if (u >= 0)
-            uid_out[(int64_t)u * nel + e] = to_d2(state[at]);
+    for (int64_t q = blockIdx.x; q < mp; q += gridDim.x) {
+        const int32_t u = q2u[q];
+        for (int e = threadIdx.x; e < nel; e += blockDim.x) {
+            const int64_t at = q * nel + wide_pos(N, e / N, e % N);
+            if (TO_STATE)
+                state[at] = from_d2<C>(u >= 0 ? uid_order[(int64_t)u * nel + e] : make_double2(0.0, 0.0));
+            else if (u >= 0)
+                uid_out[(int64_t)u * nel + e] = to_d2(state[at]);
+        }
     }
 }
 
@@ -1438,11 +1439,11 @@ void upload_state(heom_handle* h, const double* state, unsigned char* dst)
     stage.alloc((size_t)h->M * h->nel);
     HIPC(hipMemcpyAsync(stage.p, state, stage.bytes(), hipMemcpyHostToDevice, h->stream));
     const bool matrices = h->N > kMaxStates;
-    const dim3 mgrid((unsigned)h->Mp), mblock(256);
+    const dim3 mgrid(matrix_blocks(h->Mp)), mblock(kMatrixThreads);
     if (h->fp32()) {
         if (matrices)
             hipLaunchKernelGGL((copy_matrices<float2, true>), mgrid, mblock, 0, h->stream, stage.p,
-                               h->y.as<float2>(), nullptr, h->q2u.p, h->N);
+                               h->y.as<float2>(), nullptr, h->q2u.p, h->Mp, h->N);
         else
             hipLaunchKernelGGL(aos_to_soa<float2>, dim3(blocks_for(h->Mp, 256)), dim3(256), 0, h->stream, stage.p,
                                h->y.as<float2>(), h->q2u.p, h->Mp, h->N, h->paired);
@@ -1458,7 +1459,7 @@ void upload_state(heom_handle* h, const double* state, unsigned char* dst)
         double2* to = reinterpret_cast<double2*>(dst ? dst : h->y.p);
         if (matrices)
             hipLaunchKernelGGL((copy_matrices<double2, true>), mgrid, mblock, 0, h->stream, stage.p, to, nullptr,
-                               h->q2u.p, h->N);
+                               h->q2u.p, h->Mp, h->N);
         else
             hipLaunchKernelGGL(aos_to_soa<double2>, dim3(blocks_for(h->Mp, 256)), dim3(256), 0, h->stream, stage.p, to,
                                h->q2u.p, h->Mp, h->N, false);
@@ -1475,13 +1476,13 @@ void download_state(heom_handle* h, const unsigned char* src, const double2* row
     stage.alloc((size_t)h->M * h->nel);
     if (h->active < h->M)  // ADOs removed by heom_compact read back as zero
         HIPC(hipMemsetAsync(stage.p, 0, stage.bytes(), h->stream));
-    const dim3 mgrid((unsigned)h->Mp), mblock(256);
+    const dim3 mgrid(matrix_blocks(h->Mp)), mblock(kMatrixThreads);
     if (h->N > kMaxStates && h->fp32())
         hipLaunchKernelGGL((copy_matrices<float2, false>), mgrid, mblock, 0, h->stream, nullptr,
-                           reinterpret_cast<float2*>(const_cast<unsigned char*>(src)), stage.p, h->q2u.p, h->N);
+                           reinterpret_cast<float2*>(const_cast<unsigned char*>(src)), stage.p, h->q2u.p, h->Mp, h->N);
     else if (h->N > kMaxStates)
         hipLaunchKernelGGL((copy_matrices<double2, false>), mgrid, mblock, 0, h->stream, nullptr,
-                           reinterpret_cast<double2*>(const_cast<unsigned char*>(src)), stage.p, h->q2u.p, h->N);
+                           reinterpret_cast<double2*>(const_cast<unsigned char*>(src)), stage.p, h->q2u.p, h->Mp, h->N);
     else if (h->fp32())
         hipLaunchKernelGGL(soa_to_aos<float2>, dim3(blocks_for(h->Mp, 256)), dim3(256), 0, h->stream,
                            reinterpret_cast<const float2*>(src), stage.p, h->q2u.p, h->Mp, h->N, h->paired);
