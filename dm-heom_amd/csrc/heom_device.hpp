@@ -388,8 +388,9 @@ constexpr int kMatrixThreads = 256;
 constexpr unsigned matrix_blocks(int64_t mp) { return (unsigned)(mp < (1 << 20) ? mp : 1 << 20); }
 // W: bath modes
 bool wide_supported(int N, int complex_bytes, int W);
-// the largest number of wavefronts (ADOs at a time) per workgroup, a power of two <= 8
-int wide_max_ados(int N, int complex_bytes, int W);
+// the largest number of wavefronts (ADOs at a time) per workgroup, a power of two <= 8, for
+// modes that couple to at most len elements each
+int wide_max_ados(int N, int complex_bytes, bool real_h, int W, int len);
 // ados: wavefronts per workgroup, 0 = the default
 void launch_stage_wide(int N, bool real_h, int stage, const StageArgsT<double>& a, const ElementArgsT<double>& el,
                        const WideTables<double>& wt, int ados, hipStream_t s);

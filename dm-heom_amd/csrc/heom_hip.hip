@@ -1573,7 +1573,7 @@ std::vector<StageConfig> stage_candidates(heom_handle* h)
         return out;
     };
     if (h->N > kMaxStates) {
-        for (int T = wide_max_ados(h->N, (int)h->cbytes(), h->W); T >= 1; T /= 2)
+        for (int T = wide_max_ados(h->N, (int)h->cbytes(), h->real_h, h->W, h->wide_len); T >= 1; T /= 2)
             cands.push_back({HEOM_STAGE_WIDE, 1, 0, T});
     } else {
         // complex64 planes: the layout fixes the kernel family (paired: pipelined only)

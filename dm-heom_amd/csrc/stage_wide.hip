@@ -31,8 +31,7 @@ namespace heom_hip {
 
 namespace {
 
-constexpr int kWideLdsBytes = 147456;  // 144 KB of the 160 KB LDS
-constexpr int kWideLdsAll = 163840;
+constexpr int kWideLdsAll = 163840;  // LDS of a CU
 constexpr int kMaxWideStates = 32;
 // at most 8 wavefronts per workgroup, so that a lane may hold up to 256 VGPRs
 constexpr int kWideThreads = 512;
@@ -56,21 +55,6 @@ constexpr int kWideWhereBytes = 16384;
 template <typename R, int SZ, bool ONE>
 constexpr int kWideModesAhead = SZ > 24 && sizeof(R) == sizeof(double) ? (ONE ? 2 : 1) : (ONE ? 3 : 2);
 
-// the size limit of the large-system kernels (a matrix of H and T more in kWideLdsBytes,
-// with the tile's slice of the neighbour table): what a handle may ask for
-__host__ __device__ constexpr int wide_limit_bytes(int N, int cbytes, int W, int T)
-{
-    return (T + 1) * N * (N + 1) * cbytes + ((W + 2) & ~1) * T * (int)sizeof(int2);
-}
-
-int wide_tile(int N, int cbytes, int W)
-{
-    for (int T = kWideThreads / 64; T >= 1; T /= 2)
-        if (wide_limit_bytes(N, cbytes, W, T) <= kWideLdsBytes)
-            return T;
-    return 0;
-}
-
 // LDS of a workgroup of T wavefronts, in bytes: the constant matrix (H / hbar or C, complex or
 // its real part), the places by mode (where they take at most kWideWhereBytes), the "same"
 // constants (not beside 32 x 32 matrices in complex128), and a matrix per wavefront.  What lies
@@ -89,10 +73,22 @@ __host__ __device__ constexpr WideLds wide_lds(int N, int cbytes, bool real, boo
     return {h, h + g, h + g + el, h + g + el + T * cbytes * m};
 }
 // bytes of the places by mode in LDS, 0 if they stay in global memory
-int wide_where_bytes(int W, int len)
+constexpr int wide_where_bytes(int W, int len)
 {
     const int64_t b = (int64_t)W * len * 4;
     return b <= kWideWhereBytes ? (int)b : 0;
+}
+// the most wavefronts that the LDS holds the matrices of: 8 but for 32 x 32 in complex128 with
+// a complex constant matrix and many places, where it is 4
+constexpr int wide_most_waves(int N, int cbytes, bool real, int W, int len)
+{
+    const bool gam_lds = cbytes == sizeof(float2) ? kWideGamLds<float, kMaxWideStates>
+                         : N <= 24                ? kWideGamLds<double, 24>
+                                                  : kWideGamLds<double, kMaxWideStates>;
+    int T = kWideThreads / 64;
+    while (T > 1 && wide_lds(N, cbytes, real, gam_lds, T, wide_where_bytes(W, len)).total > kWideLdsAll)
+        T /= 2;
+    return T;
 }
 
 template <typename R>
@@ -831,24 +827,22 @@ struct WideShape {
     unsigned wgs;
 };
 template <typename R, int SZ>
-WideShape wide_shape(int N, bool real, int W, int len, int ntiles, int ados)
+constexpr WideShape wide_shape(int N, bool real, int W, int len, int ntiles, int ados)
 {
     const auto shape = [&](int T) {
         const int64_t all = (int64_t)(ntiles + kNumXcd - 1) / kNumXcd * kNumXcd * (kTile / T);
         const int64_t most = (int64_t)kWideCus * 4 * kWideOccupancy<R, SZ> / T;
         return WideShape{T, all <= most, (unsigned)std::min(all, most)};
     };
-    const auto lds = [&](int T) {
-        return wide_lds(N, (int)sizeof(c2<R>), real, kWideGamLds<R, SZ>, T, wide_where_bytes(W, len)).total;
-    };
-    const int fit = wide_tile(N, (int)sizeof(c2<R>), W);
+    const int fit = wide_most_waves(N, (int)sizeof(c2<R>), real, W, len);
     if (ados > 0 && ados <= fit && kTile % ados == 0)
         return shape(ados);
     // 4, as many as a CU's SIMDs; 8 where the CU's LDS does not hold two such workgroups and
     // each wavefront has several ADOs to go through (32 sites, ms per RK4 step in complex128:
     // 6,545 ADOs 0.640 with 4, 0.582 with 8; 561 ADOs 0.101 and 0.133)
     const WideShape four = shape(std::min(fit, 4));
-    return !four.one && 2 * lds(4) > kWideLdsAll && lds(8) <= kWideLdsAll ? shape(8) : four;
+    const int lds = wide_lds(N, (int)sizeof(c2<R>), real, kWideGamLds<R, SZ>, 4, wide_where_bytes(W, len)).total;
+    return !four.one && 2 * lds > kWideLdsAll && fit >= 8 ? shape(8) : four;
 }
 
 template <typename R, int SZ, bool REALH, bool ONE, bool WLDS>
@@ -919,12 +913,17 @@ void launch_ts(int N, bool real_c, const StageArgsT<double>& a, const double2* g
 
 }  // namespace
 
+// the limit on the modes of a handle: two matrices and a table entry per mode in 144 KB
 bool wide_supported(int N, int complex_bytes, int W)
 {
-    return N > kMaxStates && N <= kMaxWideStates && wide_tile(N, complex_bytes, W) > 0;
+    return N > kMaxStates && N <= kMaxWideStates &&
+           2 * (int64_t)N * (N + 1) * complex_bytes + (((int64_t)W + 2) & ~1) * 8 <= 147456;
 }
 
-int wide_max_ados(int N, int complex_bytes, int W) { return wide_tile(N, complex_bytes, W); }
+int wide_max_ados(int N, int complex_bytes, bool real_h, int W, int len)
+{
+    return wide_most_waves(N, complex_bytes, real_h, W, len);
+}
 
 void launch_stage_wide(int N, bool real_h, int stage, const StageArgsT<double>& a, const ElementArgsT<double>& el,
                        const WideTables<double>& wt, int ados, hipStream_t s)
