@@ -6,6 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <functional>
 #include <memory>
@@ -190,13 +191,13 @@ struct heom_handle {
     DevBuf<float2> pfss32, hs32, gam32;
     DevBuf<TermT<float>> terms32;
     DevBuf<heom_hip::PairTerm> pterms;  // [classes][pair_planes(N)][pair_slots]
-    // N > 8: the neighbour terms by mode (WideTables), [classes][W][wide_len]
+    // N > 8: the neighbour terms by mode (WideTables), [classes][wide_words]
     DevBuf<Term> wterms;
     DevBuf<TermT<float>> wterms32;
-    DevBuf<uint32_t> wwhere;     // then, from entry wide_place on, the places of the positions
+    DevBuf<uint32_t> wwhere;  // [classes][wide_words], then the places of the positions
     size_t wide_place = 0;
     DevBuf<int32_t> tile_order;  // tiles with plus neighbours first
-    int wide_len = 0;
+    int wide_stride = 0, wide_words = 0;
     int S = 0;                    // tier-0/1 ADOs
     std::vector<int32_t> sp_top;  // [count] tier-0/1 index of each top
     std::vector<int64_t> sp_uid;  // [S] global uid
@@ -231,10 +232,12 @@ struct heom_handle {
     heom_hip::WideTables<R> wide_tables() const
     {
         const uint16_t* places = reinterpret_cast<const uint16_t*>(wwhere.p + wide_place);
+        const heom_hip::TermT<R>* terms;
         if constexpr (sizeof(R) == sizeof(double))
-            return {wterms.p, wwhere.p, tile_order.p, places, W, wide_len};
+            terms = wterms.p;
         else
-            return {wterms32.p, wwhere.p, tile_order.p, places, W, wide_len};
+            terms = wterms32.p;
+        return {terms, wwhere.p, tile_order.p, places, W, wide_stride, wide_words};
     }
     size_t cbytes() const { return fp32() ? sizeof(float2) : sizeof(double2); }
 
@@ -271,6 +274,55 @@ void launch_stage_buffers(heom_handle* h, int stage, const void* yin, const void
 // the arguments of such a stage in FP64
 heom_hip::StageArgsT<double> stage_args64(heom_handle* h, const void* yin, const void* y0, void* pbuf, void* yout,
                                           double c1, bool reverse);
+// The terms of the elements (`per`: [classes][N*N] lists) by mode, for WideTables
+struct WideModes {
+    std::vector<heom_hip::Term> terms;  // the mode holds the element
+    std::vector<uint32_t> where;
+    int stride = 1, words = 0;
+};
+inline WideModes wide_modes(const std::vector<std::vector<heom_hip::Term>>& per, int classes, int N, int W)
+{
+    const int nel = N * N;
+    WideModes out;
+    std::vector<std::vector<heom_hip::Term>> lists((size_t)classes * W);
+    for (int cl = 0; cl < classes; ++cl) {
+        int total = W;
+        for (int e = 0; e < nel; ++e)
+            for (heom_hip::Term t : per[(size_t)cl * nel + e]) {
+                std::vector<heom_hip::Term>& list = lists[(size_t)cl * W + t.mode];
+                t.mode = e;
+                list.push_back(t);
+                out.stride = std::max(out.stride, (int)list.size());
+                ++total;
+            }
+        out.words = std::max(out.words, total);
+    }
+    if (out.stride > 64)
+        out.stride = 0;
+    else
+        out.words = W * out.stride;
+    out.terms.resize((size_t)classes * out.words);
+    out.where.assign(out.terms.size(), 0xffff0000u);
+    for (int cl = 0; cl < classes; ++cl) {
+        heom_hip::Term* terms = &out.terms[(size_t)cl * out.words];
+        uint32_t* where = &out.where[(size_t)cl * out.words];
+        int at = W;
+        for (int m = 0; m < W; ++m) {
+            const std::vector<heom_hip::Term>& list = lists[(size_t)cl * W + m];
+            if (out.stride > 0)
+                at = m * out.stride;
+            else  // an empty list starts at 0, not past the end
+                where[m] = list.empty() ? 0 : (uint32_t)at | (uint32_t)list.size() << 16;
+            for (const heom_hip::Term& t : list) {
+                const int i = t.mode / N, j = t.mode % N;
+                terms[at] = t;
+                where[at] = (uint32_t)heom_hip::wide_pos(N, i, j) | (uint32_t)(i * heom_hip::wide_pitch(N) + j) << 16;
+                ++at;
+            }
+        }
+    }
+    return out;
+}
 // builds the device layout of count instances into a fresh handle (heom_create_batch)
 void create_batch(heom_handle* h, const heom_desc* d, int count);
 // raises HEOM_E_UNSUPPORTED for `what` on a thermal-state-search handle

@@ -361,18 +361,22 @@ void launch_stage_adjoint(int N, int nterm_slots, bool real_h, int stage, const 
 // core operand reads at once fall into different banks, and one of three, so that the places
 // of a lane's elements are constants of the kernels
 __host__ __device__ constexpr int wide_pitch(int N) { return N <= 16 ? 17 : N <= 24 ? 25 : 33; }
-// The neighbour terms by mode: mode m of class c couples the elements of the terms from
-// (c * W + m) * len on, at most len of them.  `where` holds for each the element's position in
-// the state (wide_pos, low half) and its place in a matrix of row stride wide_pitch(N) (high
-// half; 0xffff in the unused entries).  tile_order: the tiles with plus neighbours, then the
-// others.
+// The neighbour terms by mode, `words` entries a class of terms and of where.  `where` holds for
+// each term the element's position in the state (wide_pos, low half) and its place in a matrix
+// of row stride wide_pitch(N) (high half).  Two forms:
+//   stride > 0   no mode couples to more than 64 elements: mode m's terms are the entries from
+//                m * stride on, stride of them (place 0xffff where the list has ended);
+//   stride = 0   some mode does: where[m] holds the number of mode m's terms (high half) and
+//                the entry of the first (low half); every list has its own length, so that the
+//                others do not take the rounds of the longest.
+// tile_order: the tiles with plus neighbours, then the others.
 template <typename R>
 struct WideTables {
     const TermT<R>* __restrict__ terms;
     const uint32_t* __restrict__ where;
     const int32_t* __restrict__ tile_order;
     const uint16_t* __restrict__ place;  // [N*N] the LDS place of every position
-    int32_t W, len;
+    int32_t W, stride, words;
 };
 // the constants of the thermal state search (tss.hip): C and (i / hbar)(E_i - E_j) per
 // instance, eps - S_u and the uid (< 0: padding, kept at zero) per slot
@@ -388,9 +392,9 @@ constexpr int kMatrixThreads = 256;
 constexpr unsigned matrix_blocks(int64_t mp) { return (unsigned)(mp < (1 << 20) ? mp : 1 << 20); }
 // W: bath modes
 bool wide_supported(int N, int complex_bytes, int W);
-// the largest number of wavefronts (ADOs at a time) per workgroup, a power of two <= 8, for
-// modes that couple to at most len elements each
-int wide_max_ados(int N, int complex_bytes, bool real_h, int W, int len);
+// the largest number of wavefronts (ADOs at a time) per workgroup, a power of two <= 8 (words:
+// of WideTables)
+int wide_max_ados(int N, int complex_bytes, bool real_h, int words);
 // ados: wavefronts per workgroup, 0 = the default
 void launch_stage_wide(int N, bool real_h, int stage, const StageArgsT<double>& a, const ElementArgsT<double>& el,
                        const WideTables<double>& wt, int ados, hipStream_t s);

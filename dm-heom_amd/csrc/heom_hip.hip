@@ -922,44 +922,28 @@ void build_pair_terms(heom_handle* h, const std::vector<std::vector<Term>>& per,
 // N > 8: the neighbour terms by mode (WideTables in heom_device.hpp)
 void build_wide_terms(heom_handle* h, const std::vector<std::vector<Term>>& per, int C)
 {
-    const int N = h->N, W = h->W, nel = N * N;
-    std::vector<std::vector<Term>> by_mode((size_t)C * W);
-    for (int cl = 0; cl < C; ++cl)
-        for (int e = 0; e < nel; ++e)
-            for (Term t : per[(size_t)cl * nel + e]) {
-                std::vector<Term>& out = by_mode[(size_t)cl * W + t.mode];
-                t.mode = e;
-                out.push_back(t);
-            }
-    size_t len = 1;
-    for (const auto& m : by_mode)
-        len = std::max(len, m.size());
-    h->wide_len = (int)len;
-    std::vector<Term> flat(by_mode.size() * len, Term{});
-    std::vector<uint32_t> where(flat.size(), 0xffff0000u);
-    for (size_t m = 0; m < by_mode.size(); ++m) {
-        std::copy(by_mode[m].begin(), by_mode[m].end(), flat.begin() + (std::ptrdiff_t)(m * len));
-        for (size_t k = 0; k < by_mode[m].size(); ++k) {
-            const int i = by_mode[m][k].mode / N, j = by_mode[m][k].mode % N;
-            where[m * len + k] = (uint32_t)wide_pos(N, i, j) | (uint32_t)(i * wide_pitch(N) + j) << 16;
-        }
-    }
-    // one allocation and copy for both: the places follow the modes' entries
+    const int N = h->N;
+    WideModes modes = wide_modes(per, C, N, h->W);
+    h->wide_stride = modes.stride;
+    h->wide_words = modes.words;
+    // one allocation and copy: the positions' places follow the modes' entries
+    std::vector<uint32_t>& where = modes.where;
     h->wide_place = where.size();
-    where.resize(where.size() + ((size_t)nel + 1) / 2);
+    where.resize(where.size() + ((size_t)h->nel + 1) / 2);
     uint16_t* place = reinterpret_cast<uint16_t*>(where.data() + h->wide_place);
     for (int i = 0; i < N; ++i)
         for (int j = 0; j < N; ++j)
             place[(size_t)wide_pos(N, i, j)] = (uint16_t)(i * wide_pitch(N) + j);
     upload(h->wwhere, where, h->stream);
     if (h->fp32()) {
-        std::vector<TermT<float>> f32(flat.size());
-        for (size_t t = 0; t < flat.size(); ++t)
-            f32[t] = {make_float2((float)flat[t].minus_c.x, (float)flat[t].minus_c.y), (float)flat[t].plus_c,
-                      flat[t].mode, flat[t].info};
+        std::vector<TermT<float>> f32(modes.terms.size());
+        for (size_t t = 0; t < f32.size(); ++t) {
+            const Term& m = modes.terms[t];
+            f32[t] = {make_float2((float)m.minus_c.x, (float)m.minus_c.y), (float)m.plus_c, m.mode, m.info};
+        }
         upload(h->wterms32, f32, h->stream);
     } else {
-        upload(h->wterms, flat, h->stream);
+        upload(h->wterms, modes.terms, h->stream);
     }
 }
 
@@ -1573,7 +1557,7 @@ std::vector<StageConfig> stage_candidates(heom_handle* h)
         return out;
     };
     if (h->N > kMaxStates) {
-        for (int T = wide_max_ados(h->N, (int)h->cbytes(), h->real_h, h->W, h->wide_len); T >= 1; T /= 2)
+        for (int T = wide_max_ados(h->N, (int)h->cbytes(), h->real_h, h->wide_words); T >= 1; T /= 2)
             cands.push_back({HEOM_STAGE_WIDE, 1, 0, T});
     } else {
         // complex64 planes: the layout fixes the kernel family (paired: pipelined only)

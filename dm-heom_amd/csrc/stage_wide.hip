@@ -73,20 +73,22 @@ __host__ __device__ constexpr WideLds wide_lds(int N, int cbytes, bool real, boo
     return {h, h + g, h + g + el, h + g + el + T * cbytes * m};
 }
 // bytes of the places by mode in LDS, 0 if they stay in global memory
-constexpr int wide_where_bytes(int W, int len)
-{
-    const int64_t b = (int64_t)W * len * 4;
-    return b <= kWideWhereBytes ? (int)b : 0;
-}
+constexpr int wide_where_bytes(int words) { return words * 4 <= kWideWhereBytes ? words * 4 : 0; }
+// whether lists of more than 64 elements (WideTables: stride = 0) have kernels of their own:
+// where the registers spill, the code of their rounds alone slows the others down (32 sites
+// with a bath each, 6,545 ADOs, complex128: 0.596 ms per RK4 step in one kernel, 0.583 apart;
+// up to 24 sites, in complex64 or with one ADO to a wavefront both take the same)
+template <typename R, int SZ, bool ONE>
+constexpr bool kWideLongApart = SZ > 24 && sizeof(R) == sizeof(double) && !ONE;
 // the most wavefronts that the LDS holds the matrices of: 8 but for 32 x 32 in complex128 with
 // a complex constant matrix and many places, where it is 4
-constexpr int wide_most_waves(int N, int cbytes, bool real, int W, int len)
+constexpr int wide_most_waves(int N, int cbytes, bool real, int words)
 {
     const bool gam_lds = cbytes == sizeof(float2) ? kWideGamLds<float, kMaxWideStates>
                          : N <= 24                ? kWideGamLds<double, 24>
                                                   : kWideGamLds<double, kMaxWideStates>;
     int T = kWideThreads / 64;
-    while (T > 1 && wide_lds(N, cbytes, real, gam_lds, T, wide_where_bytes(W, len)).total > kWideLdsAll)
+    while (T > 1 && wide_lds(N, cbytes, real, gam_lds, T, wide_where_bytes(words)).total > kWideLdsAll)
         T /= 2;
     return T;
 }
@@ -333,11 +335,13 @@ struct EdgeLanes {
 // The neighbour terms of one ADO, summed into the matrix f in LDS: for every element in the
 // order of the modes, plus before minus.  Its edges in modes m0 .. m0 + 63 are in the lanes of
 // `ed`; the modes with an edge are walked with D of them in flight (a mode that couples to
-// more than 64 elements counts as several).  Every mode makes the same loads -- through a
-// buffer resource that ends at once where the edge is missing, so that nothing is read and
-// zeros come back -- and so the wait for one mode's loads is not one for those behind it.
-// `where` is this class's, in LDS where it fits.
-template <typename R, int D>
+// more than 64 elements makes several rounds, as many as its own list needs: with all modes as
+// long as the longest, 24 sites with a bath each and one more for all of them, 3,276 ADOs, took
+// 0.441 ms per RK4 step, 0.180 so).  Every round makes the same loads -- through a buffer
+// resource that ends at once where the edge is missing, so that nothing is read and zeros come
+// back -- and so the wait for one round's loads is not one for those behind it.  `where` is
+// this class's, in LDS where it fits.
+template <typename R, int D, bool LONG>
 struct Neighbours {
     using C = c2<R>;
     using V = vec2_t<R>;
@@ -346,8 +350,9 @@ struct Neighbours {
     const TermT<R>* terms;
     const uint32_t* where;
     int64_t q;
-    int nel, lane, m0 = 0, chunk = 0, todo;
+    int nel, lane, m0 = 0, round = 0, todo;
     EdgeLanes ed;
+    uint32_t spans;  // of the modes in the lanes (stride = 0)
     uint64_t has_p, has_m, left;
     V mc[D], xp[D], xm[D];
     R pc[D];
@@ -355,7 +360,7 @@ struct Neighbours {
 
     __device__ __forceinline__ Neighbours(const StageArgsT<R>& a_, const WideTables<R>& wt_, int cls,
                                           const uint32_t* where_, EdgeLanes entries, int64_t q_, int nel_, int lane_)
-        : a(a_), wt(wt_), terms(wt_.terms + (int64_t)cls * wt_.W * wt_.len), where(where_), q(q_), nel(nel_),
+        : a(a_), wt(wt_), terms(wt_.terms + (int64_t)cls * wt_.words), where(where_), q(q_), nel(nel_),
           lane(lane_), ed(entries)
     {
         begin();
@@ -365,8 +370,16 @@ struct Neighbours {
         has_p = __ballot((int32_t)((uint32_t)ed.v.x >> 6) != a.zero_slot);
         has_m = __ballot(ed.v.y != a.zero_slot);
         left = has_p | has_m;
-        todo = __popcll(left) * ((wt.len + 63) / 64);
-        chunk = 0;
+        todo = __popcll(left);
+        if (LONG && wt.stride == 0) {
+            spans = m0 + lane < wt.W ? where[m0 + lane] : 0;
+            uint64_t longer = left;
+            for (int r = 1; longer != 0; ++r) {
+                longer &= __ballot((int)(spans >> 16) > 64 * r);
+                todo += __popcll(longer);
+            }
+        }
+        round = 0;
 #pragma unroll
         for (int u = 0; u < D; ++u)
             fetch(u);
@@ -389,19 +402,26 @@ struct Neighbours {
         const bool some = left != 0;
         const int m = some ? __builtin_ctzll(left) : 0;
         const int vx = __builtin_amdgcn_readlane(ed.v.x, m), vy = __builtin_amdgcn_readlane(ed.v.y, m);
-        const int k = chunk * 64 + lane, i = (m0 + m) * wt.len + min(k, wt.len - 1);
+        int i = (m0 + m) * wt.stride + min(lane, wt.stride - 1);
+        bool in = lane < wt.stride;
+        if (LONG && wt.stride == 0) {
+            asm volatile("");  // a branch, and no selects for the others
+            const uint32_t span = (uint32_t)__builtin_amdgcn_readlane((int)spans, m);
+            const int count = (int)(span >> 16), k = lane + 64 * round;
+            i = (int)(span & 0xffff) + max(min(k, count - 1), 0);
+            in = k < count;
+            round = (round + 1) * 64 < count ? round + 1 : 0;
+        }
+        if (!LONG || round == 0)
+            left &= left - 1;
         const uint32_t pp = where[i];
         const bool p = (has_p >> m & 1) && some, mn = (has_m >> m & 1) && some;
         xp[u] = element(p ? (int64_t)((uint32_t)vx >> 6) : 0, p, (int)(pp & 0xffff));
         xm[u] = element(mn ? (int64_t)(uint32_t)vy : 0, mn, (int)(pp & 0xffff));
         mc[u] = V{terms[i].minus_c.x, terms[i].minus_c.y};
         pc[u] = terms[i].plus_c;
-        at[u] = some && k < wt.len ? (int)(pp >> 16) : 0xffff;
+        at[u] = some && in ? (int)(pp >> 16) : 0xffff;
         n[u] = vx & 63;
-        if (++chunk * 64 >= wt.len) {
-            chunk = 0;
-            left &= left - 1;
-        }
     }
     template <bool SCALED>
     __device__ __forceinline__ void add(int u, R scale, R sq_lane, C* f)
@@ -489,7 +509,7 @@ struct Lin {
 // places by mode
 template <typename R, typename TM, int SZ, bool WLDS>
 __device__ __forceinline__ void load_constants(const c2<R>* __restrict__ m, const c2<R>* __restrict__ gam,
-                                               const uint32_t* __restrict__ where, int terms, int N, TM* ml,
+                                               const uint32_t* __restrict__ where, int words, int N, TM* ml,
                                                c2<R>* gl, uint32_t* el, bool first)
 {
     const int NP = wide_pitch(N);
@@ -522,20 +542,20 @@ __device__ __forceinline__ void load_constants(const c2<R>* __restrict__ m, cons
         }
     }
     if (WLDS)
-        for (int i0 = threadIdx.x; i0 < terms; i0 += U * step) {
+        for (int i0 = threadIdx.x; i0 < words; i0 += U * step) {
             uint32_t v[U];
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                v[u] = where[min(i0 + u * step, terms - 1)];
+                v[u] = where[min(i0 + u * step, words - 1)];
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                el[min(i0 + u * step, terms - 1)] = v[u];
+                el[min(i0 + u * step, words - 1)] = v[u];
         }
     __syncthreads();
 }
 
 // One RK4 stage (STAGE 1..4, or 0: the RHS alone) over the whole hierarchy.  N <= SZ.
-template <typename R, int SZ, int STAGE, bool REALH, bool ONE, bool WLDS>
+template <typename R, int SZ, int STAGE, bool REALH, bool ONE, bool WLDS, bool LONG>
 __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(kWideOccupancy<R, SZ>)))
 void rk4_stage_wide(StageArgsT<R> a, WideTables<R> wt, const c2<R>* __restrict__ hs_all,
                     const c2<R>* __restrict__ gam_all, int N_, int T)
@@ -557,13 +577,13 @@ void rk4_stage_wide(StageArgsT<R> a, WideTables<R> wt, const c2<R>* __restrict__
     // have no scalar registers to spare
     if (ONE)
         asm volatile("" ::"s"(a.yin), "s"(a.nb), "s"(a.mp), "s"(a.pfss), "s"(a.tile_inst), "s"(a.tile_class), "s"(wt.place),
-                     "s"(wt.where), "s"(wt.terms), "s"(wt.W), "s"(wt.len), "s"(hs_all), "s"(gam_all), "s"(N_), "s"(T),
+                     "s"(wt.where), "s"(wt.terms), "s"(wt.W), "s"(wt.stride), "s"(wt.words), "s"(hs_all), "s"(gam_all), "s"(N_), "s"(T),
                      "s"(a.zero_slot), "s"(a.ntiles), "s"(a.y0), "s"(a.yout));
     const int nel = N_ * N_;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int terms = wt.W * wt.len;
+    const int words = wt.words;
     constexpr bool GL = kWideGamLds<R, SZ>;
-    const WideLds L = wide_lds(N_, (int)sizeof(C), REALH, GL, T, WLDS ? terms * 4 : 0);
+    const WideLds L = wide_lds(N_, (int)sizeof(C), REALH, GL, T, WLDS ? words * 4 : 0);
     TM* hl = reinterpret_cast<TM*>(wide_mem);
     C* gl = reinterpret_cast<C*>(wide_mem + L.gam);
     uint32_t* el = reinterpret_cast<uint32_t*>(wide_mem + L.where);
@@ -594,9 +614,9 @@ void rk4_stage_wide(StageArgsT<R> a, WideTables<R> wt, const c2<R>* __restrict__
         const int it = a.tile_inst ? a.tile_inst[q0 / kTile] : 0;
         const int cl = tile_bath_class(a, (int)(q0 / kTile));
         const C* gam = gam_all + (int64_t)cl * nel;
-        const uint32_t* where = wt.where + (int64_t)cl * terms;
+        const uint32_t* where = wt.where + (int64_t)cl * words;
         if (it != inst || cl != cls)
-            load_constants<R, TM, SZ, WLDS>(hs_all + (int64_t)it * nel, gam, where, terms, N_, hl, gl, el, inst < 0);
+            load_constants<R, TM, SZ, WLDS>(hs_all + (int64_t)it * nel, gam, where, words, N_, hl, gl, el, inst < 0);
         inst = it;
         cls = cl;
         j += walk.gx;
@@ -629,7 +649,7 @@ void rk4_stage_wide(StageArgsT<R> a, WideTables<R> wt, const c2<R>* __restrict__
                     sig[place(k)] = own[k];
             wave_sync();
             // the first neighbours are under way during the commutator
-            Neighbours<R, kWideModesAhead<R, SZ, ONE>> nbs(a, wt, cl, WLDS ? el : where, ed, q, nel, lane);
+            Neighbours<R, kWideModesAhead<R, SZ, ONE>, LONG> nbs(a, wt, cl, WLDS ? el : where, ed, q, nel, lane);
             __builtin_amdgcn_sched_barrier(0);
 
             Product<R, NB> cm;  // sigma H - H sigma (over hbar)
@@ -709,9 +729,9 @@ __global__ __launch_bounds__(kWideThreads) void tss_iteration_wide(StageArgsT<do
     const int nel = N * N;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int terms = wt.W * wt.len;
+    const int words = wt.words;
     constexpr bool GL = kWideGamLds<double, SZ>;
-    const WideLds L = wide_lds(N, (int)sizeof(C), REALC, GL, T, WLDS ? terms * 4 : 0);
+    const WideLds L = wide_lds(N, (int)sizeof(C), REALC, GL, T, WLDS ? words * 4 : 0);
     TM* cl = reinterpret_cast<TM*>(wide_mem);
     C* gl = reinterpret_cast<C*>(wide_mem + L.gam);
     uint32_t* el = reinterpret_cast<uint32_t*>(wide_mem + L.where);
@@ -734,9 +754,9 @@ __global__ __launch_bounds__(kWideThreads) void tss_iteration_wide(StageArgsT<do
         const int it = a.tile_inst ? a.tile_inst[q0 / kTile] : 0;
         const int cc = tile_bath_class(a, (int)(q0 / kTile));
         const C* gam = gam_all + (int64_t)cc * nel;
-        const uint32_t* where = wt.where + (int64_t)cc * terms;
+        const uint32_t* where = wt.where + (int64_t)cc * words;
         if (it != inst || cc != cls)
-            load_constants<double, TM, SZ, WLDS>(ts.c + (int64_t)it * nel, gam, where, terms, N, cl, gl, el, inst < 0);
+            load_constants<double, TM, SZ, WLDS>(ts.c + (int64_t)it * nel, gam, where, words, N, cl, gl, el, inst < 0);
         inst = it;
         cls = cc;
         if (q >= a.zero_slot)
@@ -754,7 +774,7 @@ __global__ __launch_bounds__(kWideThreads) void tss_iteration_wide(StageArgsT<do
             }
         }
         wave_sync();
-        Neighbours<double, kWideModesAhead<double, SZ, true>> nbs(a, wt, cc, WLDS ? el : where, ed, q, nel, lane);
+        Neighbours<double, kWideModesAhead<double, SZ, true>, true> nbs(a, wt, cc, WLDS ? el : where, ed, q, nel, lane);
         nbs.template run<false>(1.0, sq_lane, sig);
         wave_sync();
         const C* w_ij = ts.w + (int64_t)it * nel;
@@ -827,47 +847,57 @@ struct WideShape {
     unsigned wgs;
 };
 template <typename R, int SZ>
-constexpr WideShape wide_shape(int N, bool real, int W, int len, int ntiles, int ados)
+constexpr WideShape wide_shape(int N, bool real, int words, int ntiles, int ados)
 {
     const auto shape = [&](int T) {
         const int64_t all = (int64_t)(ntiles + kNumXcd - 1) / kNumXcd * kNumXcd * (kTile / T);
         const int64_t most = (int64_t)kWideCus * 4 * kWideOccupancy<R, SZ> / T;
         return WideShape{T, all <= most, (unsigned)std::min(all, most)};
     };
-    const int fit = wide_most_waves(N, (int)sizeof(c2<R>), real, W, len);
+    const int fit = wide_most_waves(N, (int)sizeof(c2<R>), real, words);
     if (ados > 0 && ados <= fit && kTile % ados == 0)
         return shape(ados);
     // 4, as many as a CU's SIMDs; 8 where the CU's LDS does not hold two such workgroups and
     // each wavefront has several ADOs to go through (32 sites, ms per RK4 step in complex128:
     // 6,545 ADOs 0.640 with 4, 0.582 with 8; 561 ADOs 0.101 and 0.133)
     const WideShape four = shape(std::min(fit, 4));
-    const int lds = wide_lds(N, (int)sizeof(c2<R>), real, kWideGamLds<R, SZ>, 4, wide_where_bytes(W, len)).total;
+    const int lds = wide_lds(N, (int)sizeof(c2<R>), real, kWideGamLds<R, SZ>, 4, wide_where_bytes(words)).total;
     return !four.one && 2 * lds > kWideLdsAll && fit >= 8 ? shape(8) : four;
+}
+
+template <typename R, int SZ, bool REALH, bool ONE, bool WLDS, bool LONG>
+void launch_wl(int N, int stage, const StageArgsT<R>& a, const ElementArgsT<R>& el, const WideTables<R>& wt,
+               WideShape sh, hipStream_t st)
+{
+    const int T = sh.T;
+    const dim3 grid(sh.wgs), block(64 * T);
+    const size_t lds =
+        (size_t)wide_lds(N, (int)sizeof(c2<R>), REALH, kWideGamLds<R, SZ>, T, wide_where_bytes(wt.words)).total;
+    switch (stage) {
+    case 0: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 0, REALH, ONE, WLDS, LONG>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
+    case 1: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 1, REALH, ONE, WLDS, LONG>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
+    case 2: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 2, REALH, ONE, WLDS, LONG>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
+    case 3: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 3, REALH, ONE, WLDS, LONG>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
+    default: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 4, REALH, ONE, WLDS, LONG>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
+    }
 }
 
 template <typename R, int SZ, bool REALH, bool ONE, bool WLDS>
 void launch_wo(int N, int stage, const StageArgsT<R>& a, const ElementArgsT<R>& el, const WideTables<R>& wt,
                WideShape sh, hipStream_t st)
 {
-    const int T = sh.T;
-    const dim3 grid(sh.wgs), block(64 * T);
-    const size_t lds =
-        (size_t)wide_lds(N, (int)sizeof(c2<R>), REALH, kWideGamLds<R, SZ>, T, wide_where_bytes(wt.W, wt.len)).total;
-    switch (stage) {
-    case 0: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 0, REALH, ONE, WLDS>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
-    case 1: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 1, REALH, ONE, WLDS>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
-    case 2: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 2, REALH, ONE, WLDS>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
-    case 3: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 3, REALH, ONE, WLDS>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
-    default: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 4, REALH, ONE, WLDS>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
-    }
+    if (wt.stride == 0 || !kWideLongApart<R, SZ, ONE>)
+        launch_wl<R, SZ, REALH, ONE, WLDS, true>(N, stage, a, el, wt, sh, st);
+    else
+        launch_wl<R, SZ, REALH, ONE, WLDS, !kWideLongApart<R, SZ, ONE>>(N, stage, a, el, wt, sh, st);
 }
 
 template <typename R, int SZ, bool REALH>
 void launch_ws(int N, int stage, const StageArgsT<R>& a, const ElementArgsT<R>& el, const WideTables<R>& wt, int ados,
                hipStream_t st)
 {
-    const WideShape sh = wide_shape<R, SZ>(N, REALH, wt.W, wt.len, a.ntiles, ados);
-    if (wide_where_bytes(wt.W, wt.len) == 0)
+    const WideShape sh = wide_shape<R, SZ>(N, REALH, wt.words, a.ntiles, ados);
+    if (wide_where_bytes(wt.words) == 0)
         launch_wo<R, SZ, REALH, false, false>(N, stage, a, el, wt, sh, st);
     else if (sh.one)
         launch_wo<R, SZ, REALH, true, true>(N, stage, a, el, wt, sh, st);
@@ -891,8 +921,8 @@ template <int SZ, bool REALC>
 void launch_tr(int N, const StageArgsT<double>& a, const double2* gam, const WideTables<double>& wt, const WideTss& ts,
                hipStream_t st)
 {
-    const WideShape sh = wide_shape<double, SZ>(N, REALC, wt.W, wt.len, a.ntiles, 0);
-    const int wb = wide_where_bytes(wt.W, wt.len), T = sh.T;
+    const WideShape sh = wide_shape<double, SZ>(N, REALC, wt.words, a.ntiles, 0);
+    const int wb = wide_where_bytes(wt.words), T = sh.T;
     const size_t lds = (size_t)wide_lds(N, (int)sizeof(double2), REALC, kWideGamLds<double, SZ>, T, wb).total;
     const dim3 grid(sh.wgs), block(64 * T);
     if (wb)
@@ -920,9 +950,9 @@ bool wide_supported(int N, int complex_bytes, int W)
            2 * (int64_t)N * (N + 1) * complex_bytes + (((int64_t)W + 2) & ~1) * 8 <= 147456;
 }
 
-int wide_max_ados(int N, int complex_bytes, bool real_h, int W, int len)
+int wide_max_ados(int N, int complex_bytes, bool real_h, int words)
 {
-    return wide_most_waves(N, complex_bytes, real_h, W, len);
+    return wide_most_waves(N, complex_bytes, real_h, words);
 }
 
 void launch_stage_wide(int N, bool real_h, int stage, const StageArgsT<double>& a, const ElementArgsT<double>& el,
