@@ -237,7 +237,7 @@ struct heom_handle {
             terms = wterms.p;
         else
             terms = wterms32.p;
-        return {terms, wwhere.p, tile_order.p, places, W, wide_stride, wide_words};
+        return {terms, wwhere.p, tile_order.p, places, W, wide_stride, wide_words, term_slots};
     }
     size_t cbytes() const { return fp32() ? sizeof(float2) : sizeof(double2); }
 
@@ -297,10 +297,13 @@ inline WideModes wide_modes(const std::vector<std::vector<heom_hip::Term>>& per,
             }
         out.words = std::max(out.words, total);
     }
-    if (out.stride > 64)
-        out.stride = 0;
-    else
+    bool equal = true;  // (an empty list does not count)
+    for (const auto& list : lists)
+        equal = equal && (list.empty() || (list.size() + 63) / 64 == ((size_t)out.stride + 63) / 64);
+    if (equal)
         out.words = W * out.stride;
+    else
+        out.stride = 0;
     out.terms.resize((size_t)classes * out.words);
     out.where.assign(out.terms.size(), 0xffff0000u);
     for (int cl = 0; cl < classes; ++cl) {

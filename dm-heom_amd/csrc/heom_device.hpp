@@ -156,6 +156,9 @@ __host__ __device__ __forceinline__ int2 pair_slot(int N, int i, int j)
 // touch N lines for the column alone.
 //   wide_pos: the position of element (i, j) in its matrix; wide_element: the inverse
 constexpr int kWidePanel = 4;
+// up to so many states the large-system kernels read the elements' own lists of terms
+// (ElementArgsT, by position)
+constexpr int kWideListStates = 16;
 __host__ __device__ __forceinline__ int wide_pos(int N, int i, int j)
 {
     const int p = j / kWidePanel, w = N - p * kWidePanel < kWidePanel ? N - p * kWidePanel : kWidePanel;
@@ -364,11 +367,11 @@ __host__ __device__ constexpr int wide_pitch(int N) { return N <= 16 ? 17 : N <=
 // The neighbour terms by mode, `words` entries a class of terms and of where.  `where` holds for
 // each term the element's position in the state (wide_pos, low half) and its place in a matrix
 // of row stride wide_pitch(N) (high half).  Two forms:
-//   stride > 0   no mode couples to more than 64 elements: mode m's terms are the entries from
-//                m * stride on, stride of them (place 0xffff where the list has ended);
-//   stride = 0   some mode does: where[m] holds the number of mode m's terms (high half) and
-//                the entry of the first (low half); every list has its own length, so that the
-//                others do not take the rounds of the longest.
+//   stride > 0   all modes take as many rounds of 64 elements: mode m's terms are the entries
+//                from m * stride on, stride of them (place 0xffff where the list has ended);
+//   stride = 0   some take more than others: where[m] holds the number of mode m's terms (high
+//                half) and the entry of the first (low half), so that each makes the rounds of
+//                its own list and not those of the longest.
 // tile_order: the tiles with plus neighbours, then the others.
 template <typename R>
 struct WideTables {
@@ -377,6 +380,7 @@ struct WideTables {
     const int32_t* __restrict__ tile_order;
     const uint16_t* __restrict__ place;  // [N*N] the LDS place of every position
     int32_t W, stride, words;
+    int32_t slots;  // of an element's own list (ElementArgsT)
 };
 // the constants of the thermal state search (tss.hip): C and (i / hbar)(E_i - E_j) per
 // instance, eps - S_u and the uid (< 0: padding, kept at zero) per slot

@@ -1018,22 +1018,36 @@ void build_coefficients(heom_handle* h)
             dst.info = (int32_t)per[e].size() | (dst.plus_c != 0.0 ? kTermHasPlus : 0) |
                        (dst.minus_c.x != 0.0 || dst.minus_c.y != 0.0 ? kTermHasMinus : 0);
         }
-    upload(h->terms, flat, h->stream);
     upload(h->gam, gam, h->stream);
+    // the kernels for N > 8 read the lists by position, up to kWideListStates
+    const auto list = [&](size_t e) {
+        if (N <= kMaxStates)
+            return e;
+        const int2 ij = wide_element(N, (int)(e % (size_t)h->nel));
+        return e / (size_t)h->nel * (size_t)h->nel + (size_t)(ij.x * N + ij.y);
+    };
+    const size_t NT = (size_t)h->term_slots, lists = N <= kWideListStates ? flat.size() / NT : 0;
     if (h->fp32()) {
-        std::vector<TermT<float>> f32(flat.size());
-        for (size_t t = 0; t < flat.size(); ++t) {
-            f32[t].minus_c = make_float2((float)flat[t].minus_c.x, (float)flat[t].minus_c.y);
-            f32[t].plus_c = (float)flat[t].plus_c;
-            f32[t].mode = flat[t].mode;
-            f32[t].info = flat[t].info;
+        upload(h->terms, flat, h->stream);  // tier_fixup: by element
+        std::vector<TermT<float>> f32(lists * NT);
+        for (size_t t = 0; t < f32.size(); ++t) {
+            const Term& m = flat[list(t / NT) * NT + t % NT];
+            f32[t] = {make_float2((float)m.minus_c.x, (float)m.minus_c.y), (float)m.plus_c, m.mode, m.info};
         }
         std::vector<float2> g32(gam.size());
         for (size_t e = 0; e < gam.size(); ++e)
             g32[e] = make_float2((float)gam[e].x, (float)gam[e].y);
-        upload(h->terms32, f32, h->stream);
+        if (lists)
+            upload(h->terms32, f32, h->stream);
         upload(h->gam32, g32, h->stream);
         build_pair_terms(h, per, C);
+    } else if (N <= kMaxStates) {
+        upload(h->terms, flat, h->stream);
+    } else if (lists) {
+        std::vector<Term> at(flat.size());
+        for (size_t t = 0; t < at.size(); ++t)
+            at[t] = flat[list(t / NT) * NT + t % NT];
+        upload(h->terms, at, h->stream);
     }
 }
 
