@@ -114,15 +114,23 @@ struct BathClass {
 
 // The thermal state search (tss.hip): the constants of the per-ADO transform.
 struct TssState {
-    DevBuf<double2> c, ct;  // C and C^T [count][nel]
-    DevBuf<double2> w;      // (i/hbar)(E_i - E_j) [count][nel]
-    DevBuf<double2> epsm;   // eps - S_u per slot [Mp]
-    bool real_c = false;    // C has no imaginary parts (real symmetric H)
+    DevBuf<unsigned char> mem;  // holds all of the following
+    const double2 *c = nullptr, *ct = nullptr;  // C and C^T [count][nel], as far as they are read
+    const double2* w = nullptr;                 // (i/hbar)(E_i - E_j) [count][nel]
+    const double2* epsm = nullptr;              // eps - S_u per slot [Mp]
+    bool real_c = false;                        // C has no imaginary parts (real symmetric H)
     // N <= 8: the real parts of C and C^T, and the element constants in column-major order
-    DevBuf<double> cr, ctr;           // [count][nel]
-    DevBuf<double2> gam;              // [classes][N columns][N]
-    DevBuf<heom_hip::Term> terms;     // [classes][N columns][N][term slots]
-    DevBuf<int32_t> modes;            // the terms' modes alone
+    const double *cr = nullptr, *ctr = nullptr;  // [count][nel]
+    const double2* gam = nullptr;                // [classes][N columns][N]
+    const heom_hip::Term* terms = nullptr;       // [classes][N columns][N][term slots]
+    const int32_t* modes = nullptr;              // the terms' modes alone
+};
+
+// host copies of tables that create_batch uploads
+struct HostTables {
+    std::vector<int32_t> q2u;
+    std::vector<double2> gam;
+    std::vector<heom_hip::Term> terms;
 };
 
 }  // namespace heom_rt
@@ -181,7 +189,8 @@ struct heom_handle {
     std::vector<std::pair<heom_pre_evaluate_fn, void*>> pre_evaluate;
     DevBuf<int2> nb_raw, nb;                // packed neighbour table, unmasked and mask-folded
     DevBuf<int32_t> q2u, tile_inst;
-    DevBuf<int32_t> tile_plus;              // [ntiles] 1 if an ADO of the tile has a plus edge
+    DevBuf<int32_t> tile_plus;              // [ntiles] 1 if an ADO of the tile has a plus edge; N > 8:
+                                            // then [ntiles] the tiles, those with plus edges first
     DevBuf<int64_t> q_top;                  // [count] internal index of each top ADO
     DevBuf<uint8_t> mask;
     DevBuf<double2> pfss, hs, gam, mx, small;  // FP64 constants
@@ -191,12 +200,10 @@ struct heom_handle {
     DevBuf<float2> pfss32, hs32, gam32;
     DevBuf<TermT<float>> terms32;
     DevBuf<heom_hip::PairTerm> pterms;  // [classes][pair_planes(N)][pair_slots]
-    // N > 8: the neighbour terms by mode (WideTables), [classes][wide_words]
-    DevBuf<Term> wterms;
-    DevBuf<TermT<float>> wterms32;
-    DevBuf<uint32_t> wwhere;  // [classes][wide_words], then the places of the positions
-    size_t wide_place = 0;
-    DevBuf<int32_t> tile_order;  // tiles with plus neighbours first
+    // N > 8 (WideTables): the terms by mode [classes][wide_words], the elements' lists by
+    // position, where [classes][wide_words] and the places of the positions, from these bytes on
+    DevBuf<unsigned char> wide;
+    size_t wide_lists = 0, wide_where = 0, wide_place = 0;
     int wide_stride = 0, wide_words = 0;
     int S = 0;                    // tier-0/1 ADOs
     std::vector<int32_t> sp_top;  // [count] tier-0/1 index of each top
@@ -231,13 +238,17 @@ struct heom_handle {
     template <typename R>
     heom_hip::WideTables<R> wide_tables() const
     {
-        const uint16_t* places = reinterpret_cast<const uint16_t*>(wwhere.p + wide_place);
-        const heom_hip::TermT<R>* terms;
-        if constexpr (sizeof(R) == sizeof(double))
-            terms = wterms.p;
-        else
-            terms = wterms32.p;
-        return {terms, wwhere.p, tile_order.p, places, W, wide_stride, wide_words, term_slots};
+        const auto at = [&](size_t b) { return wide.p + b; };
+        using T = heom_hip::TermT<R>;
+        return {reinterpret_cast<const T*>(at(0)),
+                reinterpret_cast<const T*>(at(wide_lists)),
+                reinterpret_cast<const uint32_t*>(at(wide_where)),
+                tile_plus.p + ntiles,
+                reinterpret_cast<const uint16_t*>(at(wide_place)),
+                W,
+                wide_stride,
+                wide_words,
+                term_slots};
     }
     size_t cbytes() const { return fp32() ? sizeof(float2) : sizeof(double2); }
 
@@ -326,8 +337,9 @@ inline WideModes wide_modes(const std::vector<std::vector<heom_hip::Term>>& per,
     }
     return out;
 }
-// builds the device layout of count instances into a fresh handle (heom_create_batch)
-void create_batch(heom_handle* h, const heom_desc* d, int count);
+// builds the device layout of count instances into a fresh handle (heom_create_batch); `host`
+// receives the tables
+void create_batch(heom_handle* h, const heom_desc* d, int count, HostTables* host = nullptr);
 // raises HEOM_E_UNSUPPORTED for `what` on a thermal-state-search handle
 void reject_tss(heom_handle* h, const char* what);
 // nsteps RK4 steps of the handle's state (through the captured step graph when enabled)

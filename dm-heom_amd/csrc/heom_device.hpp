@@ -156,8 +156,7 @@ __host__ __device__ __forceinline__ int2 pair_slot(int N, int i, int j)
 // touch N lines for the column alone.
 //   wide_pos: the position of element (i, j) in its matrix; wide_element: the inverse
 constexpr int kWidePanel = 4;
-// up to so many states the large-system kernels read the elements' own lists of terms
-// (ElementArgsT, by position)
+// up to so many states the large-system kernels read the elements' own lists of terms too
 constexpr int kWideListStates = 16;
 __host__ __device__ __forceinline__ int wide_pos(int N, int i, int j)
 {
@@ -376,11 +375,12 @@ __host__ __device__ constexpr int wide_pitch(int N) { return N <= 16 ? 17 : N <=
 template <typename R>
 struct WideTables {
     const TermT<R>* __restrict__ terms;
+    const TermT<R>* __restrict__ lists;  // [classes][N*N][slots] by position, N <= kWideListStates
     const uint32_t* __restrict__ where;
     const int32_t* __restrict__ tile_order;
     const uint16_t* __restrict__ place;  // [N*N] the LDS place of every position
     int32_t W, stride, words;
-    int32_t slots;  // of an element's own list (ElementArgsT)
+    int32_t slots;  // of an element's own list
 };
 // the constants of the thermal state search (tss.hip): C and (i / hbar)(E_i - E_j) per
 // instance, eps - S_u and the uid (< 0: padding, kept at zero) per slot

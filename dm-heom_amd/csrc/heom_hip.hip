@@ -510,12 +510,12 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(NT <= 2
     }
 }
 
-
 }  // namespace
-
 
 namespace heom_rt {
 
+// h may go at once: a copy from memory that is not pinned is synchronous for the host
+// (hipMemcpyAsync's note in hip_runtime_api.h)
 template <typename T>
 void upload(DevBuf<T>& d, const std::vector<T>& h, hipStream_t s)
 {
@@ -791,15 +791,12 @@ void build_tile_plus(heom_handle* h, const std::vector<int2>& nb)
         for (int64_t q = 0; q < h->Mp; ++q)
             if ((int32_t)((uint32_t)nb[(size_t)m * h->Mp + q].x >> 6) != h->zero_slot)
                 f[(size_t)(q / kTile)] = 1;
-    upload(h->tile_plus, f, h->stream);
-    if (h->N > kMaxStates) {
-        std::vector<int32_t> order;
+    if (h->N > kMaxStates)  // the order of WideTables behind the flags
         for (int want = 1; want >= 0; --want)
             for (int t = 0; t < h->ntiles; ++t)
                 if (f[(size_t)t] == want)
-                    order.push_back(t);
-        upload(h->tile_order, order, h->stream);
-    }
+                    f.push_back(t);
+    upload(h->tile_plus, f, h->stream);
 }
 
 // the bath class of each tile, by its instance (only where the classes differ)
@@ -919,35 +916,31 @@ void build_pair_terms(heom_handle* h, const std::vector<std::vector<Term>>& per,
     upload(h->pterms, flat, h->stream);
 }
 
-// N > 8: the neighbour terms by mode (WideTables in heom_device.hpp)
-void build_wide_terms(heom_handle* h, const std::vector<std::vector<Term>>& per, int C)
+// N > 8: the tables of WideTables; `lists`: the elements' terms, [classes][N*N][slots] by position
+template <typename R>
+void build_wide_terms(heom_handle* h, const std::vector<std::vector<Term>>& per, int C, const std::vector<Term>& lists)
 {
     const int N = h->N;
-    WideModes modes = wide_modes(per, C, N, h->W);
+    const WideModes modes = wide_modes(per, C, N, h->W);
     h->wide_stride = modes.stride;
     h->wide_words = modes.words;
-    // one allocation and copy: the positions' places follow the modes' entries
-    std::vector<uint32_t>& where = modes.where;
-    h->wide_place = where.size();
-    where.resize(where.size() + ((size_t)h->nel + 1) / 2);
-    uint16_t* place = reinterpret_cast<uint16_t*>(where.data() + h->wide_place);
+    h->wide_lists = modes.terms.size() * sizeof(TermT<R>);
+    h->wide_where = h->wide_lists + lists.size() * sizeof(TermT<R>);
+    h->wide_place = h->wide_where + modes.where.size() * sizeof(uint32_t);
+    std::vector<unsigned char> mem(h->wide_place + (size_t)h->nel * sizeof(uint16_t));
+    TermT<R>* out = reinterpret_cast<TermT<R>*>(mem.data());
+    for (const auto* from : {&modes.terms, &lists})
+        for (const Term& t : *from)
+            *out++ = {mk2<R>((R)t.minus_c.x, (R)t.minus_c.y), (R)t.plus_c, t.mode, t.info};
+    std::memcpy(mem.data() + h->wide_where, modes.where.data(), modes.where.size() * sizeof(uint32_t));
+    uint16_t* place = reinterpret_cast<uint16_t*>(mem.data() + h->wide_place);
     for (int i = 0; i < N; ++i)
         for (int j = 0; j < N; ++j)
             place[(size_t)wide_pos(N, i, j)] = (uint16_t)(i * wide_pitch(N) + j);
-    upload(h->wwhere, where, h->stream);
-    if (h->fp32()) {
-        std::vector<TermT<float>> f32(modes.terms.size());
-        for (size_t t = 0; t < f32.size(); ++t) {
-            const Term& m = modes.terms[t];
-            f32[t] = {make_float2((float)m.minus_c.x, (float)m.minus_c.y), (float)m.plus_c, m.mode, m.info};
-        }
-        upload(h->wterms32, f32, h->stream);
-    } else {
-        upload(h->wterms, modes.terms, h->stream);
-    }
+    upload(h->wide, mem, h->stream);
 }
 
-void build_coefficients(heom_handle* h)
+void build_coefficients(heom_handle* h, HostTables* host)
 {
     const int N = h->N, W = h->W, C = (int)h->classes.size();
     std::vector<std::vector<Term>> per((size_t)C * N * N);
@@ -1002,8 +995,6 @@ void build_coefficients(heom_handle* h)
     if (N <= kMaxStates ? !stage_supported(N, most) : most > 8)
         raise(HEOM_E_UNSUPPORTED, "more than 8 neighbour terms per matrix element");
     h->term_slots = stage_term_slots(most);
-    if (N > kMaxStates)
-        build_wide_terms(h, per, C);
     // pad every element's list; padding terms read table column W, which always
     // holds the zero slot
     std::vector<Term> flat((size_t)C * N * N * h->term_slots);
@@ -1019,35 +1010,41 @@ void build_coefficients(heom_handle* h)
                        (dst.minus_c.x != 0.0 || dst.minus_c.y != 0.0 ? kTermHasMinus : 0);
         }
     upload(h->gam, gam, h->stream);
-    // the kernels for N > 8 read the lists by position, up to kWideListStates
-    const auto list = [&](size_t e) {
-        if (N <= kMaxStates)
-            return e;
-        const int2 ij = wide_element(N, (int)(e % (size_t)h->nel));
-        return e / (size_t)h->nel * (size_t)h->nel + (size_t)(ij.x * N + ij.y);
-    };
-    const size_t NT = (size_t)h->term_slots, lists = N <= kWideListStates ? flat.size() / NT : 0;
+    if (N <= kMaxStates || h->fp32())  // N > 8: read by tier_fixup alone
+        upload(h->terms, flat, h->stream);
+    if (N > kMaxStates) {
+        std::vector<Term> lists;
+        if (N <= kWideListStates)
+            for (int e = 0; e < C * N * N; ++e) {
+                const int2 ij = wide_element(N, e % (N * N));
+                const auto from = flat.begin() + (std::ptrdiff_t)(e / (N * N) * N * N + ij.x * N + ij.y) * h->term_slots;
+                lists.insert(lists.end(), from, from + h->term_slots);
+            }
+        if (h->fp32())
+            build_wide_terms<float>(h, per, C, lists);
+        else
+            build_wide_terms<double>(h, per, C, lists);
+    }
     if (h->fp32()) {
-        upload(h->terms, flat, h->stream);  // tier_fixup: by element
-        std::vector<TermT<float>> f32(lists * NT);
-        for (size_t t = 0; t < f32.size(); ++t) {
-            const Term& m = flat[list(t / NT) * NT + t % NT];
-            f32[t] = {make_float2((float)m.minus_c.x, (float)m.minus_c.y), (float)m.plus_c, m.mode, m.info};
-        }
         std::vector<float2> g32(gam.size());
         for (size_t e = 0; e < gam.size(); ++e)
             g32[e] = make_float2((float)gam[e].x, (float)gam[e].y);
-        if (lists)
-            upload(h->terms32, f32, h->stream);
         upload(h->gam32, g32, h->stream);
+        if (N <= kMaxStates) {
+            std::vector<TermT<float>> f32(flat.size());
+            for (size_t t = 0; t < flat.size(); ++t) {
+                f32[t].minus_c = make_float2((float)flat[t].minus_c.x, (float)flat[t].minus_c.y);
+                f32[t].plus_c = (float)flat[t].plus_c;
+                f32[t].mode = flat[t].mode;
+                f32[t].info = flat[t].info;
+            }
+            upload(h->terms32, f32, h->stream);
+        }
         build_pair_terms(h, per, C);
-    } else if (N <= kMaxStates) {
-        upload(h->terms, flat, h->stream);
-    } else if (lists) {
-        std::vector<Term> at(flat.size());
-        for (size_t t = 0; t < at.size(); ++t)
-            at[t] = flat[list(t / NT) * NT + t % NT];
-        upload(h->terms, at, h->stream);
+    }
+    if (host) {
+        host->gam = std::move(gam);
+        host->terms = std::move(flat);
     }
 }
 
@@ -1234,7 +1231,7 @@ void setup_tiers(heom_handle* h, const heom_desc* d, const std::vector<std::vect
     }
 }
 
-void create_batch(heom_handle* h, const heom_desc* d, int count)
+void create_batch(heom_handle* h, const heom_desc* d, int count, HostTables* host)
 {
     for (int k = 0; k < count; ++k)
         validate(&d[k]);
@@ -1407,7 +1404,7 @@ void create_batch(heom_handle* h, const heom_desc* d, int count)
     h->norms.alloc(h->M);
     h->mx.alloc((size_t)count * h->nel);
     h->small.alloc((size_t)count * h->nel);
-    build_coefficients(h);
+    build_coefficients(h, host);
     h->paired = use_paired_layout(h);
     const size_t plane = h->paired ? (size_t)pair_planes(N) * Mp * 2 * sizeof(float2)
                                    : (size_t)N * N * Mp * h->cbytes();
@@ -1427,6 +1424,8 @@ void create_batch(heom_handle* h, const heom_desc* d, int count)
     if (h->fp32())
         setup_tiers(h, d, u2q_all);
     choose_stage_kernel(h);
+    if (host)
+        host->q2u = std::move(q2u);
     HIPC(hipStreamSynchronize(h->stream));
 }
 
@@ -2252,7 +2251,20 @@ int heom_device_bytes(heom_handle* h, int64_t* bytes)
         if (!bytes)
             raise(HEOM_E_INVALID, "bytes is NULL");
         int64_t b = h->y.bytes() + h->pbuf.bytes() + h->ya.bytes() + h->yb.bytes();
-        b += h->wterms.bytes() + h->wterms32.bytes() + h->wwhere.bytes() + h->tile_order.bytes();
+        b += h->wide.bytes() + h->tile_plus.bytes() + h->tile_class.bytes() + h->inst_class_d.bytes() +
+             h->pterms.bytes() + h->fscratch.bytes();
+        for (const auto& x : h->extra)
+            b += x->bytes();
+        if (h->tss)
+            b += h->tss->mem.bytes();
+        if (h->adj) {
+            const AdjointState& a = *h->adj;
+            for (const auto* x : {&a.cps, &a.traj, &a.seg, &a.f2, &a.f3, &a.f4, &a.lam, &a.a, &a.b, &a.c})
+                b += x->bytes();
+            for (const auto* x : {&a.hs, &a.gam, &a.pfss, &a.part, &a.gs, &a.src})
+                b += x->bytes();
+            b += a.terms.bytes();
+        }
         for (auto* x : {&h->pfss, &h->hs, &h->gam, &h->mx, &h->small, &h->y64, &h->sa64, &h->sb64, &h->p64,
                         &h->sp_pfss, &h->sp_tmp})
             b += x->bytes();

@@ -632,7 +632,7 @@ __device__ __forceinline__ void load_constants(const c2<R>* __restrict__ m, cons
 template <typename R, int SZ, int STAGE, bool REALH, bool ONE, bool WLDS, bool LONG, bool BYEL>
 __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(kWideOccupancy<R, SZ>)))
 void rk4_stage_wide(StageArgsT<R> a, WideTables<R> wt, const c2<R>* __restrict__ hs_all,
-                    const c2<R>* __restrict__ gam_all, const TermT<R>* __restrict__ lists, int N_, int T)
+                    const c2<R>* __restrict__ gam_all, int N_, int T)
 {
     using C = c2<R>;
     using TM = std::conditional_t<REALH, R, C>;
@@ -652,7 +652,7 @@ void rk4_stage_wide(StageArgsT<R> a, WideTables<R> wt, const c2<R>* __restrict__
     if (ONE)
         asm volatile("" ::"s"(a.yin), "s"(a.nb), "s"(a.mp), "s"(a.pfss), "s"(a.tile_inst), "s"(a.tile_class), "s"(wt.place),
                      "s"(wt.where), "s"(wt.terms), "s"(wt.W), "s"(wt.stride), "s"(wt.words), "s"(hs_all), "s"(gam_all), "s"(N_), "s"(T),
-                     "s"(lists), "s"(wt.slots), "s"(a.zero_slot), "s"(a.ntiles), "s"(a.y0), "s"(a.yout));
+                     "s"(wt.slots), "s"(a.zero_slot), "s"(a.ntiles), "s"(a.y0), "s"(a.yout));
     const int nel = N_ * N_;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int words = wt.words;
@@ -749,7 +749,7 @@ void rk4_stage_wide(StageArgsT<R> a, WideTables<R> wt, const c2<R>* __restrict__
             __builtin_amdgcn_sched_barrier(0);
             operand();  // the neighbour terms cover it
             if (BYEL && wt.W <= 64 && by_element(nbs.todo, NL, wt.slots))
-                add_by_element<LINEAR && !APART, R, NL>(a, lists + (int64_t)cl * nel * wt.slots, wt.slots, wt.W, ed.v,
+                add_by_element<LINEAR && !APART, R, NL>(a, wt.lists + (int64_t)cl * nel * wt.slots, wt.slots, wt.W, ed.v,
                                                         nel, lane, a.c1, sq_lane, place, sig);
             else
                 nbs.template run<LINEAR && !APART>(a.c1, sq_lane, sig);
@@ -954,11 +954,11 @@ void launch_wl(int N, int stage, const StageArgsT<R>& a, const ElementArgsT<R>& 
     const size_t lds =
         (size_t)wide_lds(N, (int)sizeof(c2<R>), REALH, kWideGamLds<R, SZ>, T, wide_where_bytes(wt.words)).total;
     switch (stage) {
-    case 0: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 0, REALH, ONE, WLDS, LONG, BYEL>), grid, block, lds, st, a, wt, el.hs, el.gam, el.terms, N, T); break;
-    case 1: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 1, REALH, ONE, WLDS, LONG, BYEL>), grid, block, lds, st, a, wt, el.hs, el.gam, el.terms, N, T); break;
-    case 2: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 2, REALH, ONE, WLDS, LONG, BYEL>), grid, block, lds, st, a, wt, el.hs, el.gam, el.terms, N, T); break;
-    case 3: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 3, REALH, ONE, WLDS, LONG, BYEL>), grid, block, lds, st, a, wt, el.hs, el.gam, el.terms, N, T); break;
-    default: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 4, REALH, ONE, WLDS, LONG, BYEL>), grid, block, lds, st, a, wt, el.hs, el.gam, el.terms, N, T); break;
+    case 0: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 0, REALH, ONE, WLDS, LONG, BYEL>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
+    case 1: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 1, REALH, ONE, WLDS, LONG, BYEL>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
+    case 2: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 2, REALH, ONE, WLDS, LONG, BYEL>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
+    case 3: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 3, REALH, ONE, WLDS, LONG, BYEL>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
+    default: hipLaunchKernelGGL((rk4_stage_wide<R, SZ, 4, REALH, ONE, WLDS, LONG, BYEL>), grid, block, lds, st, a, wt, el.hs, el.gam, N, T); break;
     }
 }
 

@@ -23,6 +23,9 @@
 #include <algorithm>
 #include <cmath>
 #include <complex>
+#include <cstring>
+#include <functional>
+#include <type_traits>
 #include <vector>
 
 #include "handle.hpp"
@@ -239,11 +242,11 @@ void launch_iteration_t(heom_handle* h, const TssArgs& a)
     const TssState& T = *h->tss;
     const dim3 grid(h->ntiles), block(64 * N);
     if (T.real_c)
-        hipLaunchKernelGGL((tss_iteration<N, NT, double>), grid, block, 0, h->stream, a, T.gam.p, T.terms.p, T.modes.p,
-                           T.cr.p, T.ctr.p, T.w.p);
+        hipLaunchKernelGGL((tss_iteration<N, NT, double>), grid, block, 0, h->stream, a, T.gam, T.terms, T.modes, T.cr,
+                           T.ctr, T.w);
     else
-        hipLaunchKernelGGL((tss_iteration<N, NT, double2>), grid, block, 0, h->stream, a, T.gam.p, T.terms.p,
-                           T.modes.p, T.c.p, T.ct.p, T.w.p);
+        hipLaunchKernelGGL((tss_iteration<N, NT, double2>), grid, block, 0, h->stream, a, T.gam, T.terms, T.modes,
+                           T.c, T.ct, T.w);
 }
 
 template <int N>
@@ -329,7 +332,8 @@ int heom_create_tss_batch(const heom_desc* descs, int32_t count, const double* c
             d[(size_t)k].pf_same_sum = pss[(size_t)k].data();
         }
         h = new heom_handle();
-        create_batch(h, d.data(), count);
+        HostTables host;
+        create_batch(h, d.data(), count, &host);
         auto T = std::make_unique<TssState>();
         std::vector<double2> cv((size_t)count * nel), ctv((size_t)count * nel), wv((size_t)count * nel);
         for (int k = 0; k < count; ++k) {
@@ -349,12 +353,9 @@ int heom_create_tss_batch(const heom_desc* descs, int32_t count, const double* c
                 }
         }
         // eps - S_u per slot, in the handle's ADO order (q2u holds batch-global uids)
-        std::vector<int32_t> q2u((size_t)h->Mp);
-        HIPC(hipMemcpyAsync(q2u.data(), h->q2u.p, q2u.size() * sizeof(int32_t), hipMemcpyDeviceToHost, h->stream));
-        HIPC(hipStreamSynchronize(h->stream));
         std::vector<double2> em((size_t)h->Mp, make_double2(eps.real(), eps.imag()));
         for (int64_t q = 0; q < h->Mp; ++q) {
-            const int32_t u = q2u[(size_t)q];
+            const int32_t u = host.q2u[(size_t)q];
             if (u < 0)
                 continue;
             const int k = (int)(std::upper_bound(h->inst_u.begin(), h->inst_u.end(), (int64_t)u) - h->inst_u.begin()) - 1;
@@ -362,50 +363,60 @@ int heom_create_tss_batch(const heom_desc* descs, int32_t count, const double* c
             em[(size_t)q] = make_double2(eps.real() - descs[k].pf_same_sum[2 * lu],
                                          eps.imag() - descs[k].pf_same_sum[2 * lu + 1]);
         }
-        auto up = [&](auto& b, const auto& v) {  // complete on return: v may be a temporary
-            b.alloc(v.size());
-            HIPC(hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, h->stream));
-            HIPC(hipStreamSynchronize(h->stream));
-        };
         T->real_c = true;
         for (const double2& x : cv)
             T->real_c = T->real_c && x.y == 0.0;
-        up(T->c, cv);
-        up(T->ct, ctv);
+        // one allocation and one copy for what the iteration's kernel reads
+        std::vector<unsigned char> mem;
+        std::vector<std::function<void()>> places;
+        auto add = [&](auto& place, const auto& v) {
+            const size_t at = (mem.size() + 15) / 16 * 16, bytes = v.size() * sizeof(v[0]);
+            mem.resize(at + bytes);
+            std::memcpy(mem.data() + at, v.data(), bytes);
+            places.push_back([&place, at, t = T.get()] {
+                place = reinterpret_cast<std::decay_t<decltype(place)>>(t->mem.p + at);
+            });
+        };
+        add(T->w, wv);
+        add(T->epsm, em);
+        if (N > kMaxStates || !T->real_c)
+            add(T->c, cv);
         if (N <= kMaxStates) {
-            // real parts of C and C^T, and the element constants in column-major order
-            // (a wavefront of the iteration kernel evaluates one column)
-            std::vector<double> cr(cv.size()), ctr(cv.size());
-            for (size_t e = 0; e < cv.size(); ++e) {
-                cr[e] = cv[e].x;
-                ctr[e] = ctv[e].x;
+            if (T->real_c) {
+                std::vector<double> cr(cv.size()), ctr(cv.size());
+                for (size_t e = 0; e < cv.size(); ++e) {
+                    cr[e] = cv[e].x;
+                    ctr[e] = ctv[e].x;
+                }
+                add(T->cr, cr);
+                add(T->ctr, ctr);
+            } else {
+                add(T->ct, ctv);
             }
+            // the element constants in column-major order (a wavefront of the iteration kernel
+            // evaluates one column)
             const int NT = h->term_slots, classes = (int)h->classes.size();
-            std::vector<double2> gam((size_t)classes * nel), gam_c(gam.size());
-            std::vector<Term> terms((size_t)classes * nel * NT), terms_c(terms.size());
+            std::vector<double2> gam(host.gam.size());
+            std::vector<Term> terms(host.terms.size());
             std::vector<int32_t> modes(terms.size());
-            HIPC(hipMemcpyAsync(gam.data(), h->gam.p, gam.size() * sizeof(double2), hipMemcpyDeviceToHost, h->stream));
-            HIPC(hipMemcpyAsync(terms.data(), h->terms.p, terms.size() * sizeof(Term), hipMemcpyDeviceToHost,
-                                h->stream));
-            HIPC(hipStreamSynchronize(h->stream));
             for (int cl = 0; cl < classes; ++cl)
                 for (int i = 0; i < N; ++i)
                     for (int j = 0; j < N; ++j) {
                         const size_t from = (size_t)cl * nel + i * N + j, to = (size_t)cl * nel + j * N + i;
-                        gam_c[to] = gam[from];
+                        gam[to] = host.gam[from];
                         for (int k = 0; k < NT; ++k) {
-                            terms_c[to * NT + k] = terms[from * NT + k];
-                            modes[to * NT + k] = terms[from * NT + k].mode;
+                            terms[to * NT + k] = host.terms[from * NT + k];
+                            modes[to * NT + k] = host.terms[from * NT + k].mode;
                         }
                     }
-            up(T->cr, cr);
-            up(T->ctr, ctr);
-            up(T->gam, gam_c);
-            up(T->terms, terms_c);
-            up(T->modes, modes);
+            add(T->gam, gam);
+            add(T->terms, terms);
+            add(T->modes, modes);
         }
-        up(T->w, wv);
-        up(T->epsm, em);
+        T->mem.alloc(mem.size());
+        HIPC(hipMemcpyAsync(T->mem.p, mem.data(), mem.size(), hipMemcpyHostToDevice, h->stream));
+        for (const auto& place : places)
+            place();
         HIPC(hipStreamSynchronize(h->stream));
         h->tss = std::move(T);
     });
@@ -436,7 +447,7 @@ int heom_tss_step(heom_handle* h, int64_t n)
         for (int64_t s = 0; s < n; ++s) {
             if (N <= kMaxStates) {
                 // y -> ya, then the two exchange their places
-                const TssArgs a{h->y.as<double2>(), h->ya.as<double2>(), h->nb.p, h->pfss.p, T.epsm.p, h->q2u.p, ti,
+                const TssArgs a{h->y.as<double2>(), h->ya.as<double2>(), h->nb.p, h->pfss.p, T.epsm, h->q2u.p, ti,
                                 h->tile_plus.p, h->uniform ? nullptr : h->tile_class.p, h->Mp, h->ntiles,
                                 h->zero_slot, h->xcd_chunk};
                 switch (N) {
@@ -456,7 +467,7 @@ int heom_tss_step(heom_handle* h, int64_t n)
             }
             const StageArgsT<double> a = stage_args64(h, h->y.p, h->y.p, h->pbuf.p, h->ya.p, 0.0, false);
             launch_tss_wide(N, T.real_c, a, h->gam.p, h->wide_tables<double>(),
-                            WideTss{T.c.p, T.w.p, T.epsm.p, h->q2u.p}, h->stream);
+                            WideTss{T.c, T.w, T.epsm, h->q2u.p}, h->stream);
             HIPC(hipGetLastError());
             std::swap(h->y.p, h->ya.p);
             h->timing.rhs_launches += 1;
