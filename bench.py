@@ -389,9 +389,9 @@ def norms_run(calls: int = 12) -> dict:
 
 
 def tss_run(host, iterations: int = 20) -> dict:
-    """Thermal state search iterations (heom_tss_step: one f_TSS evaluation by the stage
-    kernel plus the per-ADO eigenbasis transform) on the same hierarchy, timed on the
-    host around a synchronised run of `iterations` iterations."""
+    """Thermal state search iterations (heom_tss_step: one kernel each, f_TSS and the per-ADO
+    eigenbasis transform; it has to read and write the state once) on the same hierarchy,
+    timed on the host around a synchronised run of `iterations` iterations."""
     import time
 
     h = host.create_tss_handle()
@@ -404,10 +404,10 @@ def tss_run(host, iterations: int = 20) -> dict:
     top = h.get_top()
     h.close()
     nel = host.states * host.states
-    transform_bytes = 2.0 * host.matrices * nel * 16
+    alg_bytes = 2.0 * host.matrices * nel * 16
     return {"workload": f"thermal state search on the {host.matrices}-ADO hierarchy, {iterations} iterations",
             "ms_per_iteration": per * 1e3, "ado_iterations_per_s": host.matrices / per,
-            "transform_alg_bytes": transform_bytes,
+            "alg_bytes_per_iteration": alg_bytes,
             "top_trace_minus_1": float(abs(np.trace(top) - 1.0))}
 
 

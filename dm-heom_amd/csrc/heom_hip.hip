@@ -202,10 +202,10 @@ __global__ __launch_bounds__(64) void observe_tops(const double2* __restrict__ t
 // hierarchy_norm (dm-heom/cl/heom/hierarchy_norm.cl:15-45): one workgroup per 64-ADO tile,
 // lane = ADO (so every load is a coalesced plane segment), the tile's physical planes
 // dealt round-robin to kNormWaves wavefronts, whose partial sums wavefront 0 adds in a
-// fixed order.  A 16-byte slot of the paired complex64 layout holds two elements; the
-// squares of all its components are summed.  Splitting the planes keeps small hierarchies
-// of large matrices (20,475 ADOs of 24 x 24 at 576 planes) from running one long serial
-// loop per thread on a few waves per CU.
+// fixed order (N <= kMaxStates; matrix-major states: hierarchy_norm_matrices).  A 16-byte
+// slot of the paired complex64 layout holds two elements; the squares of all its components
+// are summed.  Splitting the planes keeps small hierarchies from running one serial loop of
+// up to 64 planes per thread on a few waves per CU.
 constexpr int kNormWaves = 8;
 
 template <typename V>

@@ -17,11 +17,14 @@
 // The wavefronts of a workgroup share only H / hbar and the "same" constants in LDS, so there
 // is a barrier only where the instance changes; the LDS accesses of one wavefront complete
 // in order.
+// An ADO of many edges in a launch of one ADO to a wavefront adds its terms with the elements in
+// the lanes instead (add_by_element, up to 16 sites).
 // Measured at 24 sites, 20,475 ADOs (ms per RK4 step; before: workgroups of 4 ADOs on element
 // planes, every element's term list with a missing neighbour's zeros read as well): 1.008 ->
-// 0.668 in complex128, 0.697 -> 0.449 in complex64; at 9 sites, 715 ADOs, 0.0280 -> 0.0266.  A
-// wavefront's own instructions bound it (some 400 cycles an edge), not memory: the state's 12
-// passes take 0.451 and 0.225 ms at the rate of a large copy.
+// 0.668 in complex128, 0.697 -> 0.449 in complex64; at 9 sites, 55 ADOs, 0.0250 -> 0.0207.  A
+// complex128 step moves 3.2 GB between the L2 and the fabric at 4.7 TB/s (a large copy: 5.0), 2.3 GB
+// of it the state's 12 passes and the rest neighbours that miss the L2; in complex64 it is 1.7 GB
+// at 3.9 TB/s.  The two or three wavefronts of a SIMD wait 40% of their cycles for loads and LDS.
 #include <algorithm>
 #include <type_traits>
 
